@@ -205,26 +205,30 @@ struct XYLds {
 template <int NQ, typename S>
 __device__ __forceinline__ void cell_states(int lim, const S* __restrict__ lp, int ps, int at, int stride, S up[NQ],
                                             S dn[NQ]) {
+  with_limiter(lim, [&](auto L) {
 #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    const S p = lp[q * ps + at];
-    const S s = lim_average(lim, p - lp[q * ps + at - stride], lp[q * ps + at + stride] - p);
-    up[q] = p + s * S(0.5);
-    dn[q] = p - s * S(0.5);
-  }
+    for (int q = 0; q < NQ; q++) {
+      const S p = lp[q * ps + at];
+      const S s = lim_average<L.value>(p - lp[q * ps + at - stride], lp[q * ps + at + stride] - p);
+      up[q] = p + s * S(0.5);
+      dn[q] = p - s * S(0.5);
+    }
+  });
 }
 
 // One of the two: the upper state when `up` holds, else the lower.
 template <int NQ, typename S>
 __device__ __forceinline__ void cell_state(int lim, const S* __restrict__ lp, int ps, int at, int stride, bool up,
                                            S v[NQ]) {
+  with_limiter(lim, [&](auto L) {
 #pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    const S p = lp[q * ps + at];
-    const S s = lim_average(lim, p - lp[q * ps + at - stride], lp[q * ps + at + stride] - p);
-    const S hs = s * S(0.5);
-    v[q] = up ? p + hs : p - hs;
-  }
+    for (int q = 0; q < NQ; q++) {
+      const S p = lp[q * ps + at];
+      const S s = lim_average<L.value>(p - lp[q * ps + at - stride], lp[q * ps + at + stride] - p);
+      const S hs = s * S(0.5);
+      v[q] = up ? p + hs : p - hs;
+    }
+  });
 }
 
 // y faces exchange slots (1,2) and (5,6) when `ydir` holds (axis_perm<1>
@@ -854,8 +858,10 @@ __device__ __forceinline__ void z_body(const Box<S>& b, unsigned lb, double dt, 
     take(pm);
     fetch(k0);
     take(pc);
+    with_limiter(lim, [&](auto L) {
 #pragma unroll
-    for (int q = 0; q < NQ; q++) pu[q] = pm[q] + lim_average(lim, pm[q] - p0[q], pc[q] - pm[q]) * S(0.5);
+      for (int q = 0; q < NQ; q++) pu[q] = pm[q] + lim_average<L.value>(pm[q] - p0[q], pc[q] - pm[q]) * S(0.5);
+    });
     fetch(k0 + 1);
   } else {
     fetch(k0 - 1);
@@ -909,12 +915,17 @@ __device__ __forceinline__ void z_body(const Box<S>& b, unsigned lb, double dt, 
     }
     S left[NQ], right[NQ];
     if constexpr (ORDER == 2) {
+      with_limiter(lim, [&](auto L) {
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+          const S s = lim_average<L.value>(pc[q] - pm[q], pn[q] - pc[q]);
+          left[q] = pu[q];
+          right[q] = pc[q] - s * S(0.5);
+          pu[q] = pc[q] + s * S(0.5);
+        }
+      });
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
-        const S s = lim_average(lim, pc[q] - pm[q], pn[q] - pc[q]);
-        left[q] = pu[q];
-        right[q] = pc[q] - s * S(0.5);
-        pu[q] = pc[q] + s * S(0.5);
         pm[q] = pc[q];
         pc[q] = pn[q];
       }
@@ -1080,13 +1091,15 @@ __device__ __forceinline__ void slab_body(const Box<S>& b, unsigned lb, double d
     if constexpr (ORDER == 2) {
       S p1[NQ];
       wget(tid, slot1, p1);
+      with_limiter(lim, [&](auto L) {
 #pragma unroll
-      for (int q = 0; q < NQ; q++) {
-        const S sl = lim_average(lim, p1[q] - lo[q], nx[q] - p1[q]);
-        left[q] = pu[q];
-        right[q] = p1[q] - sl * S(0.5);
-        pu[q] = p1[q] + sl * S(0.5);
-      }
+        for (int q = 0; q < NQ; q++) {
+          const S sl = lim_average<L.value>(p1[q] - lo[q], nx[q] - p1[q]);
+          left[q] = pu[q];
+          right[q] = p1[q] - sl * S(0.5);
+          pu[q] = p1[q] + sl * S(0.5);
+        }
+      });
     } else {
 #pragma unroll
       for (int q = 0; q < NQ; q++) {
@@ -1137,8 +1150,10 @@ __device__ __forceinline__ void slab_body(const Box<S>& b, unsigned lb, double d
         take(ur, f, pa, col, k0 - 1);      // P(k0-1)
         fetch(col, k0, ur, f);
         take(ur, f, pb, col, k0);          // P(k0)
+        with_limiter(lim, [&](auto L) {
 #pragma unroll
-        for (int q = 0; q < NQ; q++) pu[q] = pa[q] + lim_average(lim, pa[q] - p0[q], pb[q] - pa[q]) * S(0.5);
+          for (int q = 0; q < NQ; q++) pu[q] = pa[q] + lim_average<L.value>(pa[q] - p0[q], pb[q] - pa[q]) * S(0.5);
+        });
         wput(tid, k0 & 1, pb);
         fetch(col, k0 + 1, ur, f);
         take(ur, f, p0, col, k0 + 1);      // P(k0+1)

@@ -184,55 +184,61 @@ __device__ __forceinline__ T cfastX(const Phys& ph, const T p[8]) {
 }
 
 // average() of the slope limiters, src/hydro_core.f90:735-796
-template <typename T>
-__device__ __forceinline__ T lim_average(int lim, T a, T b) {
+template <int LIM, typename T>
+__device__ __forceinline__ T lim_average(T a, T b) {
   using A = Ar<T>;
-  T s, c, d;
-  switch (lim) {
-    case LIM_NO_LIMIT:
-      return T(0.5) * (a + b);
-    case LIM_MINMOD:
-      s = sign1(a);
-      return s * dmax(T(0), dmin(tabs(a), s * b));
-    case LIM_VAN_LEER:
-      if (a * b <= T(0)) return T(0);
-      return A::div((a * b) * (a + b), a * a + b * b);
-    case LIM_VAN_ALBADA: {
-      const T delta = T(1e-7);
-      return A::div(a * (b * b + delta) + b * (a * a + delta), (a * a + b * b) + delta);
-    }
-    case LIM_UMIST:
-      s = sign1(a);
-      c = T(0.25) * a + T(0.75) * b;
-      d = T(0.75) * a + T(0.25) * b;
-      return s * dmax(T(0), dmin(dmin(dmin(T(2) * tabs(a), (T(2) * s) * b), s * c), s * d));
-    case LIM_WOODWARD:
-      s = sign1(a);
-      c = T(0.5) * (a + b);
-      return s * dmax(T(0), dmin(dmin(T(2) * tabs(a), (T(2) * s) * b), s * c));
-    case LIM_SUPERBEE: {
-      s = sign1(b);
-      const T av1 = dmin(T(2) * tabs(b), s * a);
-      const T av2 = dmin(tabs(b), (T(2) * s) * a);
-      return s * dmax(dmax(T(0), av1), av2);
-    }
-    default:  // LIM_NO_AVERAGE
-      return T(0);
+  if constexpr (LIM == LIM_NO_LIMIT) {
+    return T(0.5) * (a + b);
+  } else if constexpr (LIM == LIM_MINMOD) {
+    const T s = sign1(a);
+    return s * dmax(T(0), dmin(tabs(a), s * b));
+  } else if constexpr (LIM == LIM_VAN_LEER) {
+    if (a * b <= T(0)) return T(0);
+    return A::div((a * b) * (a + b), a * a + b * b);
+  } else if constexpr (LIM == LIM_VAN_ALBADA) {
+    const T delta = T(1e-7);
+    return A::div(a * (b * b + delta) + b * (a * a + delta), (a * a + b * b) + delta);
+  } else if constexpr (LIM == LIM_UMIST) {
+    const T s = sign1(a);
+    const T c = T(0.25) * a + T(0.75) * b;
+    const T d = T(0.75) * a + T(0.25) * b;
+    return s * dmax(T(0), dmin(dmin(dmin(T(2) * tabs(a), (T(2) * s) * b), s * c), s * d));
+  } else if constexpr (LIM == LIM_WOODWARD) {
+    const T s = sign1(a);
+    const T c = T(0.5) * (a + b);
+    return s * dmax(T(0), dmin(dmin(T(2) * tabs(a), (T(2) * s) * b), s * c));
+  } else if constexpr (LIM == LIM_SUPERBEE) {
+    const T s = sign1(b);
+    const T av1 = dmin(T(2) * tabs(b), s * a);
+    const T av2 = dmin(tabs(b), (T(2) * s) * a);
+    return s * dmax(dmax(T(0), av1), av2);
+  } else {  // LIM_NO_AVERAGE
+    return T(0);
   }
 }
 
-// limiter, src/hydro_core.f90:712-731 (in place on pl, pr)
-template <int NQ = 8, typename T>
-__device__ __forceinline__ void limiter(int lim, const T pll[NQ], T pl[NQ], T pr[NQ], const T prr[NQ]) {
-#pragma unroll
-  for (int q = 0; q < NQ; q++) {
-    const T dl = pl[q] - pll[q];
-    const T dm = pr[q] - pl[q];
-    const T dr = prr[q] - pr[q];
-    const T al = lim_average(lim, dl, dm);
-    const T ar = lim_average(lim, dm, dr);
-    pl[q] = pl[q] + al * T(0.5);
-    pr[q] = pr[q] - ar * T(0.5);
+// One dispatch on the run's limiter around a whole reconstruction: f gets
+// the limiter as a compile-time constant, f(lim_c<LIM>).  Dispatched inside
+// lim_average instead, the branch chain ran once per variable and cell and
+// kept the compiler from overlapping one variable's LDS reads with the next
+// one's arithmetic: at 256^3 the FP64 xy corrector took 1240 us against 1160
+// with one dispatch (mixed 620 against 555), the slab corrector at
+// 128x128x4 30 us against 26.
+template <int LIM>
+struct lim_c {
+  static constexpr int value = LIM;
+};
+template <typename F>
+__device__ __forceinline__ void with_limiter(int lim, F&& f) {
+  switch (lim) {
+    case LIM_MINMOD: f(lim_c<LIM_MINMOD>()); break;
+    case LIM_NO_LIMIT: f(lim_c<LIM_NO_LIMIT>()); break;
+    case LIM_VAN_LEER: f(lim_c<LIM_VAN_LEER>()); break;
+    case LIM_VAN_ALBADA: f(lim_c<LIM_VAN_ALBADA>()); break;
+    case LIM_UMIST: f(lim_c<LIM_UMIST>()); break;
+    case LIM_WOODWARD: f(lim_c<LIM_WOODWARD>()); break;
+    case LIM_SUPERBEE: f(lim_c<LIM_SUPERBEE>()); break;
+    default: f(lim_c<LIM_NO_AVERAGE>()); break;
   }
 }
 
