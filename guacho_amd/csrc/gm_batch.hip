@@ -135,6 +135,7 @@ gm::Box<S> box_view(const Slot& s, int slot) {
   gm::Box<S> b;
   b.g = geom_of(s.p);
   b.ph.cv = s.p.cv;
+  b.ph.rcv = 1.0 / s.p.cv;
   b.ph.gamma = s.p.gamma;
   b.ph.mhd = s.p.mhd ? 1 : 0;
   b.ph.pmhd = s.p.pmhd ? 1 : 0;

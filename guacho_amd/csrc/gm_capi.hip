@@ -637,6 +637,7 @@ void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, unsigned char* scr
   b.g.gmem = 0;
   b.g.npas = p.neq - 8;
   b.ph.cv = p.cv;
+  b.ph.rcv = 1.0 / p.cv;
   b.ph.gamma = p.gamma;
   b.ph.mhd = p.mhd ? 1 : 0;
   b.ph.pmhd = p.pmhd ? 1 : 0;
@@ -708,6 +709,7 @@ int gm_create(const gm_params* params, gm_ctx** out) {
   g.gmem = 0;
   g.npas = params->neq - 8;
   c->ph.cv = params->cv;
+  c->ph.rcv = 1.0 / params->cv;
   c->ph.gamma = params->gamma;
   c->ph.mhd = params->mhd ? 1 : 0;
   c->ph.pmhd = params->pmhd ? 1 : 0;

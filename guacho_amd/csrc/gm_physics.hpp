@@ -25,17 +25,24 @@ namespace gm {
 // depends).  FP32 -- the mixed form's
 // reconstruction and fluxes -- uses the hardware reciprocal and square
 // root (v_rcp_f32, v_sqrt_f32, about 1 ulp), since its accuracy is measured
-// against the FP64 path by tolerance.
+// against the FP64 path by tolerance.  div_by(a, b, recip(b)) is div(a, b)
+// for a denominator that is nonzero and finite: without v_div_fixup, and
+// with the reciprocal in hand wherever one denominator serves several
+// divisions or is chosen between two that each already have theirs.
 template <typename T>
 struct Ar;
 template <>
 struct Ar<double> {
   static __device__ __forceinline__ double div(double a, double b) { return gm_div(a, b); }
+  static __device__ __forceinline__ double recip(double b) { return gm_recip(b); }
+  static __device__ __forceinline__ double div_by(double a, double b, double r) { return gm_div_by(a, b, r); }
   static __device__ __forceinline__ double sqrt(double a) { return gm_sqrt(a); }
 };
 template <>
 struct Ar<float> {
   static __device__ __forceinline__ float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+  static __device__ __forceinline__ float recip(float b) { return __builtin_amdgcn_rcpf(b); }
+  static __device__ __forceinline__ float div_by(float a, float, float r) { return a * r; }
   static __device__ __forceinline__ float sqrt(float a) { return __builtin_amdgcn_sqrtf(a); }
 };
 
@@ -49,6 +56,7 @@ enum : int {
 // Physical constants of a run, uniform across a launch.
 struct Phys {
   double cv, gamma;
+  double rcv;      // 1 / cv
   int mhd, pmhd;   // full MHD / passive B
   int limiter;
   int eos;         // GM_EOS_ADIABATIC, GM_EOS_SINGLE_SPECIE or GM_EOS_H_RATE
@@ -86,7 +94,7 @@ __device__ __forceinline__ void axis_perm(T v[8]) {
 // densities (:86-90); EOS_H_RATE reads the first one (the neutral density).
 template <int NQ = 8>
 __device__ __forceinline__ void u2prim(const Phys& ph, const double u[NQ], double p[NQ]) {
-  gm_u2prim(ph.cv, ph.mhd, u, p);
+  gm_u2prim_rcv(ph.cv, ph.rcv, ph.mhd, u, p);
 #pragma unroll
   for (int a = 8; a < NQ; a++) p[a] = u[a];
   if (ph.eos == GM_EOS_SINGLE_SPECIE || (NQ > 8 && ph.eos == GM_EOS_H_RATE)) (void)gm_eos(ph.eos, ph.tempsc, p);
@@ -95,7 +103,7 @@ __device__ __forceinline__ void u2prim(const Phys& ph, const double u[NQ], doubl
 // ... and u2prim's temperature T (:90-112).
 template <int NQ = 8>
 __device__ __forceinline__ double u2prim_t(const Phys& ph, const double u[NQ], double p[NQ]) {
-  gm_u2prim(ph.cv, ph.mhd, u, p);
+  gm_u2prim_rcv(ph.cv, ph.rcv, ph.mhd, u, p);
 #pragma unroll
   for (int a = 8; a < NQ; a++) p[a] = u[a];
   return gm_eos(NQ > 8 ? ph.eos : (ph.eos == GM_EOS_H_RATE ? GM_EOS_ADIABATIC : ph.eos), ph.tempsc, p);
@@ -160,7 +168,7 @@ __device__ __forceinline__ void prim2f(const Phys& ph, const T p[NQ], T f[NQ]) {
 // csound, src/hydro_core.f90:544-553
 template <typename T>
 __device__ __forceinline__ T csound(const Phys& ph, T pr, T d) {
-  return Ar<T>::sqrt(Ar<T>::div((T)ph.gamma * pr, d));
+  return Ar<T>::sqrt(Ar<T>::div_by((T)ph.gamma * pr, d, Ar<T>::recip(d)));
 }
 
 // one component of cfast, src/hydro_core.f90:576-579 (the CFL candidates;
@@ -169,7 +177,7 @@ template <typename T>
 __device__ __forceinline__ T cfast1(T g, T pr, T d, T b2, T bn) {
   using A = Ar<T>;
   const T t = g * pr + b2;
-  return A::sqrt(A::div(T(0.5) * (t + A::sqrt(t * t - (((T(4) * g) * pr) * bn) * bn)), d));
+  return A::sqrt(A::div_by(T(0.5) * (t + A::sqrt(t * t - (((T(4) * g) * pr) * bn) * bn)), d, A::recip(d)));
 }
 
 // cfastX, src/hydro_core.f90:591-604
@@ -178,9 +186,10 @@ __device__ __forceinline__ T cfastX(const Phys& ph, const T p[8]) {
   using A = Ar<T>;
   const T g = (T)ph.gamma;
   const T b2 = (p[5] * p[5] + p[6] * p[6]) + p[7] * p[7];
-  const T cs2va2 = A::div(g * p[4] + b2, p[0]);
-  return A::sqrt(T(0.5) * (cs2va2 + A::sqrt(cs2va2 * cs2va2
-                                             - A::div(A::div(((T(4) * g) * p[4]) * (p[5] * p[5]), p[0]), p[0]))));
+  const T ri = A::recip(p[0]);
+  const T cs2va2 = A::div_by(g * p[4] + b2, p[0], ri);
+  const T q = A::div_by(A::div_by(((T(4) * g) * p[4]) * (p[5] * p[5]), p[0], ri), p[0], ri);
+  return A::sqrt(T(0.5) * (cs2va2 + A::sqrt(cs2va2 * cs2va2 - q)));
 }
 
 // average() of the slope limiters, src/hydro_core.f90:735-796
@@ -255,10 +264,11 @@ __device__ __forceinline__ void hlld_star_side(const T s[8], T bx, T smu, T smsM
     byst = T(0);
     bzst = T(0);
   } else {
-    vst = s[2] - A::div((bx * s[6]) * sMmu, den);
-    wst = s[3] - A::div((bx * s[7]) * sMmu, den);
-    byst = A::div(s[6] * (s[0] * (smu * smu) - bx * bx), den);
-    bzst = A::div(s[7] * (s[0] * (smu * smu) - bx * bx), den);
+    const T ri = A::recip(den);
+    vst = s[2] - A::div_by((bx * s[6]) * sMmu, den, ri);
+    wst = s[3] - A::div_by((bx * s[7]) * sMmu, den, ri);
+    byst = A::div_by(s[6] * (s[0] * (smu * smu) - bx * bx), den, ri);
+    bzst = A::div_by(s[7] * (s[0] * (smu * smu) - bx * bx), den, ri);
   }
 }
 
@@ -295,15 +305,17 @@ __device__ __forceinline__ bool hlld_cs(const Phys& ph, const T pl[NQ], const T 
   const T slmul = sl - pl[1], srmur = sr - pr[1];
   const T rholul = pl[0] * pl[1], rhorur = pr[0] * pr[1];
   const T den_m = srmur * pr[0] - slmul * pl[0];
-  const T sM = A::div(((srmur * rhorur - slmul * rholul) - ptr) + ptl, den_m);
+  const T rden_m = A::recip(den_m);
+  const T sM = A::div_by(((srmur * rhorur - slmul * rholul) - ptr) + ptl, den_m, rden_m);
   const T srmsM = sr - sM, slmsM = sl - sM;
-  const T rhostl = A::div(pl[0] * slmul, slmsM);
-  const T rhostr = A::div(pr[0] * srmur, srmsM);
+  const T rl = A::recip(slmsM), rr = A::recip(srmsM);
+  const T rhostl = A::div_by(pl[0] * slmul, slmsM, rl);
+  const T rhostr = A::div_by(pr[0] * srmur, srmsM, rr);
   const T sqrl = A::sqrt(rhostl), sqrr = A::sqrt(rhostr);
   const T sstl = sM - A::div(tabs(bx), sqrl);
   const T sstr = sM + A::div(tabs(bx), sqrr);
-  const T pst = A::div(((srmur * pr[0]) * ptl - (slmul * pl[0]) * ptr)
-                       + (((pl[0] * pr[0]) * srmur) * slmul) * (pr[1] - pl[1]), den_m);
+  const T pst = A::div_by(((srmur * pr[0]) * ptl - (slmul * pl[0]) * ptr)
+                          + (((pl[0] * pr[0]) * srmur) * slmul) * (pr[1] - pl[1]), den_m, rden_m);
 
   T vstl, wstl, bystl, bzstl, vstr, wstr, bystr, bzstr;
   hlld_star_side(pl, bx, slmul, slmsM, sM - pl[1], vstl, wstl, bystl, bzstl);
@@ -325,16 +337,17 @@ __device__ __forceinline__ bool hlld_cs(const Phys& ph, const T pl[NQ], const T 
   const T e = hlld_energy(cv, s, bx);
   const T vdotb = (s[1] * bx + s[2] * s[6]) + s[3] * s[7];
   const T vstdotbst = (sM * bx + vst * byst) + wst * bzst;
-  const T est = A::div(((smu * e - pt * s[1]) + pst * sM) + bx * (vdotb - vstdotbst), smsM);
+  const T rs = A::recip(smsM);
+  const T est = A::div_by(((smu * e - pt * s[1]) + pst * sM) + bx * (vdotb - vstdotbst), smsM, rs);
 
   T vt = vst, wt = wst, byt = byst, bzt = bzst, et = est, vdb = vstdotbst;
   if (!single) {
-    const T dd = sqrl + sqrr;
-    const T vstst = A::div((sqrl * vstl + sqrr * vstr) + (bystr - bystl) * signbx, dd);
-    const T wstst = A::div((sqrl * wstl + sqrr * wstr) + (bzstr - bzstl) * signbx, dd);
+    const T dd = sqrl + sqrr, rd = A::recip(dd);
+    const T vstst = A::div_by((sqrl * vstl + sqrr * vstr) + (bystr - bystl) * signbx, dd, rd);
+    const T wstst = A::div_by((sqrl * wstl + sqrr * wstr) + (bzstr - bzstl) * signbx, dd, rd);
     const T sqlr = A::sqrt(rhostl * rhostr);
-    const T bystst = A::div((sqrl * bystr + sqrr * bystl) + (sqlr * (vstr - vstl)) * signbx, dd);
-    const T bzstst = A::div((sqrl * bzstr + sqrr * bzstl) + (sqlr * (wstr - wstl)) * signbx, dd);
+    const T bystst = A::div_by((sqrl * bystr + sqrr * bystl) + (sqlr * (vstr - vstl)) * signbx, dd, rd);
+    const T bzstst = A::div_by((sqrl * bzstr + sqrr * bzstl) + (sqlr * (wstr - wstl)) * signbx, dd, rd);
     const T vststdotbstst = (sM * bx + vstst * bystst) + wstst * bzstst;
     // eL** = eL* - sqrt(rhoL*)(...)signBx ; eR** = eR* + sqrt(rhoR*)(...)signBx
     const T corr = (sqr * (vstdotbst - vststdotbstst)) * signbx;
@@ -356,7 +369,7 @@ __device__ __forceinline__ bool hlld_cs(const Phys& ph, const T pl[NQ], const T 
   // passive scalars of the flux side, one expression for its star and
   // double-star regions (hlld.f90:149-151, 197-199, 276-278, 307-309)
 #pragma unroll
-  for (int a = 8; a < NQ; a++) ff[a] = A::div((sM * s[a]) * smu, smsM);
+  for (int a = 8; a < NQ; a++) ff[a] = A::div_by((sM * s[a]) * smu, smsM, rs);
   return true;
 }
 
@@ -373,8 +386,9 @@ __device__ __forceinline__ void hll_average(const Phys& ph, const T pl[NQ], cons
   prim2f<NQ>(ph, pr, fr);
   prim2u<NQ>(ph, pl, ul);
   prim2u<NQ>(ph, pr, ur);
+  const T w = sr - sl, ri = Ar<T>::recip(w);
 #pragma unroll
-  for (int q = 0; q < NQ; q++) ff[q] = Ar<T>::div((sr * fl[q] - sl * fr[q]) + (sl * sr) * (ur[q] - ul[q]), sr - sl);
+  for (int q = 0; q < NQ; q++) ff[q] = Ar<T>::div_by((sr * fl[q] - sl * fr[q]) + (sl * sr) * (ur[q] - ul[q]), w, ri);
 }
 
 // prim2fhlle, src/hlle.f90:48-83
@@ -424,11 +438,12 @@ __device__ __forceinline__ bool hllc_cs(const Phys& ph, const T pl[NQ], const T 
   uuk[1] = rhost * sst;
   uuk[2] = rhost * s[2];
   uuk[3] = rhost * s[3];
-  uuk[4] = rhost * (A::div(ek, s[0]) + (sst - s[1]) * (sst + A::div(s[4], s[0] * smu)));
+  const T ri = A::recip(s[0]);
+  uuk[4] = rhost * (A::div_by(ek, s[0], ri) + (sst - s[1]) * (sst + A::div(s[4], s[0] * smu)));
 #pragma unroll
-  for (int q = 5; q < 8; q++) uuk[q] = ph.pmhd ? A::div(rhost * s[q], s[0]) : T(0);
+  for (int q = 5; q < 8; q++) uuk[q] = ph.pmhd ? A::div_by(rhost * s[q], s[0], ri) : T(0);
 #pragma unroll
-  for (int a = 8; a < NQ; a++) uuk[a] = A::div(rhost * s[a], s[0]);  // hllc.f90:94-97, 123-126
+  for (int a = 8; a < NQ; a++) uuk[a] = A::div_by(rhost * s[a], s[0], ri);  // hllc.f90:94-97, 123-126
   prim2f<NQ>(ph, s, ff);
   prim2u<NQ>(ph, s, uu);
 #pragma unroll
