@@ -76,7 +76,7 @@ struct gm_batch {
   unsigned tiles[gm::KC_COUNT] = {0};
   bool tables_dirty = true;
   bool graph_dirty = true;
-  gm::Shape shape = {256, 16};
+  gm::Shape shape = {256, 16, 16, 0, 0};
   bool tuned = false;
   double tuned_ms = 0.0;
   hipGraph_t graph = nullptr;
@@ -86,7 +86,7 @@ struct gm_batch {
   // the same geometry reuse it
   int cap_nbox = -1;
   unsigned cap_tiles[gm::KC_COUNT] = {0};
-  gm::Shape cap_shape = {0, 0};
+  gm::Shape cap_shape{};
   bool cap_sources = false;
   bool cap_viscous = false;
   int cap_neq = 0;
@@ -224,7 +224,7 @@ void enqueue_steps_t(gm_batch* b, int nsteps, int tuning) {
   hipStream_t s = b->stream;
   const gm::Shape& sh = b->shape;
   const int solver = b->bp.riemann_solver, fcd = b->bp.enable_flux_cd;
-  const unsigned txy = b->tiles[gm::KC_XY], tcol = b->tiles[gm::KC_COL], tslab = b->tiles[gm::KC_SLAB];
+  const unsigned txy = b->tiles[gm::KC_XY], tcol = b->tiles[gm::KC_COL], tfld = b->tiles[gm::KC_FIELD], tslab = b->tiles[gm::KC_SLAB];
   const int npas = b->neq - 8;
   // With flux-CD and no source or viscous pass, each box's CFL minimum for
   // the next step is folded into the corrector's field update (its clock
@@ -234,7 +234,7 @@ void enqueue_steps_t(gm_batch* b, int nsteps, int tuning) {
   for (int st = 0; st < nsteps; st++) {
     if (!fold) {
       gm::launch_clock_begin(s, b->dclk, b->dslots, n);
-      gm::launch_cfl_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, b->derr, sh, npas);
+      gm::launch_cfl_batch(s, boxes, pre(gm::KC_FIELD), n, tfld, b->dclk, b->derr, sh, npas);
     }
     gm::launch_clock_dt(s, b->dclk, b->dslots, n, tuning);
     for (int stage = 1; stage <= 2; stage++) {
@@ -244,12 +244,12 @@ void enqueue_steps_t(gm_batch* b, int nsteps, int tuning) {
         gm::launch_xy_batch(s, boxes, pre(gm::KC_XY), n, txy, b->dclk, stage, solver, fcd, b->derr, npas);
         gm::launch_z_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, stage, solver, fcd, b->derr, sh, npas);
       }
-      if (fold && stage == 2) gm::launch_bfield_cfl_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, b->derr, sh, npas);
-      else if (fcd) gm::launch_bfield_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, stage, sh);
-      if (b->any_sources) gm::launch_sources_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, stage, sh);
+      if (fold && stage == 2) gm::launch_bfield_cfl_batch(s, boxes, pre(gm::KC_FIELD), n, tfld, b->dclk, b->derr, sh, npas);
+      else if (fcd) gm::launch_bfield_batch(s, boxes, pre(gm::KC_FIELD), n, tfld, b->dclk, stage, sh);
+      if (b->any_sources) gm::launch_sources_batch(s, boxes, pre(gm::KC_FIELD), n, tfld, b->dclk, stage, sh);
       // viscous_copy (src/hydro_solver.f90:188) after the corrector
       if (stage == 2 && b->any_viscous)
-        gm::launch_viscous_batch(s, boxes, pre(gm::KC_COL), n, tcol, b->dclk, sh);
+        gm::launch_viscous_batch(s, boxes, pre(gm::KC_FIELD), n, tfld, b->dclk, sh);
     }
   }
 }
@@ -284,7 +284,7 @@ bool graph_matches(const gm_batch* b) {
          b->cap_viscous == b->any_viscous && b->cap_neq == b->neq &&
          b->cap_shape.block == b->shape.block && b->cap_shape.slab == b->shape.slab &&
          b->cap_shape.slab_both == b->shape.slab_both &&
-         b->cap_shape.kchunk == b->shape.kchunk && std::memcmp(b->cap_tiles, b->tiles, sizeof b->tiles) == 0;
+         b->cap_shape.kchunk == b->shape.kchunk && b->cap_shape.fchunk == b->shape.fchunk && std::memcmp(b->cap_tiles, b->tiles, sizeof b->tiles) == 0;
 }
 
 // Time candidate shapes on the admitted boxes; keep the fastest: the
@@ -324,10 +324,10 @@ int autotune(gm_batch* b) {
   for (int sl : slabs)
     for (int blk : blocks)
       for (int kc : chunks)
-        if (rc == GM_OK) rc = time_shape(gm::Shape{blk, kc, sl, 0});
+        if (rc == GM_OK) rc = time_shape(gm::Shape{blk, kc, kc, sl, 0});
   const gm::Shape cols = best_sh;
   for (int sl : both_slabs)
-    if (rc == GM_OK) rc = time_shape(gm::Shape{cols.block, cols.kchunk, sl, 1});
+    if (rc == GM_OK) rc = time_shape(gm::Shape{cols.block, cols.kchunk, cols.fchunk, sl, 1});
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc != GM_OK) return rc;
@@ -584,8 +584,8 @@ int gm_batch_add(gm_batch* b, const gm_params* p, const double* u, double cfl, d
   BHIP(b, hipMemcpyAsync(b->dclk + slot, &c, sizeof(gm::BoxClock), hipMemcpyHostToDevice, x));
   // the first step's CFL minimum (get_timestep over the uploaded state),
   // which the batch's field update folds in for every later step
-  if (b->esize == 8) gm::launch_cfl(x, box_view<double>(s, slot), &b->dclk[slot].dtmin, b->derr, gm::Shape{256, 16});
-  else gm::launch_cfl(x, box_view<float>(s, slot), &b->dclk[slot].dtmin, b->derr, gm::Shape{256, 16});
+  if (b->esize == 8) gm::launch_cfl_clock(x, box_view<double>(s, slot), &b->dclk[slot].dtmin, b->derr, gm::column_shape(g));
+  else gm::launch_cfl_clock(x, box_view<float>(s, slot), &b->dclk[slot].dtmin, b->derr, gm::column_shape(g));
   BHIP(b, hipGetLastError());
   BHIP(b, hipStreamSynchronize(x));
   s.used = true;

@@ -40,20 +40,18 @@ const char* const kTableCoolCond =
     "table cooling (GM_COOL_DMC / GM_COOL_CHI) with thermal conduction is not built: the reference's conduction "
     "then starts from the half-step temperature of the interior cells";
 
+// device scalars: the kernels' error bits and the working space of the
+// launch-wide minima
 struct Scalars {
-  unsigned long long dtmin;
-  unsigned long long tcmin;  // conduction: min rho / Ksp(T) (bits of a positive double)
+  gm::MinRed red;
   int err;
-  int pad;
 };
-
-__global__ void k_init_dtmin(Scalars* s) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) s->dtmin = (unsigned long long)__double_as_longlong(1e30);
-}
-
-__global__ void k_init_tcmin(Scalars* s) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) s->tcmin = (unsigned long long)__double_as_longlong(1.79769313486231570815e+308);
-}
+// what the kernels publish to the host, in pinned memory
+struct HostScalars {
+  double dtmin;  // get_timestep's minimum
+  double tcmin;  // conduction: min rho / Ksp(T)
+  int err;
+};
 
 __global__ void k_clear_err(Scalars* s) {
   if (threadIdx.x == 0 && blockIdx.x == 0) s->err = 0;
@@ -75,7 +73,7 @@ struct gm_ctx {
   void* Ssrc = nullptr;  // the user source plugin's s of a stage (neq doubles per cell)
   void* Dl = nullptr;    // staging of the Temp / divB downloads (one double per cell), on first use
   Scalars* dscal = nullptr;  // device scalars
-  Scalars* hscal = nullptr;  // pinned host mirror
+  HostScalars* hscal = nullptr;
   bool ghosts_dirty = true;
   // the last gm_tstep reduced the CFL minimum of its result into hscal and
   // nothing has changed U's interior or the EOS since
@@ -94,7 +92,7 @@ struct gm_ctx {
   gm::Cooling cool{};                   // kind 0: no cooling
   gm::Conduction cond{};                // kind 0: no thermal conduction
   int tc_substeps = 0;                  // sub-steps of the last step's conduction
-  gm::Shape shape = {256, 16};  // tile width, z-pencil length
+  gm::Shape shape{};
   // planes per slab of the 2.5-D stage kernel, per stage (predictor,
   // corrector); 0: the two-kernel stage (xy plane tiles, then z pencils
   // through W)
@@ -452,14 +450,10 @@ template <typename S>
 void conduction_t(gm_ctx* c, const gm::Box<S>& b, double dt) {
   const gm::Conduction& tc = c->cond;
   timed(c, KC_CONDUCTION, [&] {
-    hipLaunchKernelGGL(k_init_tcmin, dim3(1), dim3(1), 0, c->stream, c->dscal);
-    gm::launch_tc_dtmin(c->stream, b, tc, &c->dscal->tcmin);
+    gm::launch_tc_dtmin(c->stream, b, tc, gm::MinOut{&c->dscal->red, &c->hscal->tcmin, nullptr, nullptr, 0});
   });
-  (void)hipMemcpyAsync(&c->hscal->tcmin, &c->dscal->tcmin, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                       c->stream);
   (void)hipStreamSynchronize(c->stream);
-  double dtp;
-  std::memcpy(&dtp, &c->hscal->tcmin, sizeof dtp);
+  const double dtp = c->hscal->tcmin;
   double ddx = c->p.dx < c->p.dy ? c->p.dx : c->p.dy;
   ddx = ddx < c->p.dz ? ddx : c->p.dz;
   const double x = ddx * tc.rsc;
@@ -488,6 +482,11 @@ void conduction_t(gm_ctx* c, const gm::Box<S>& b, double dt) {
       gm::launch_tc_substep(c->stream, b, tc, dts);
     }
   });
+}
+
+// get_timestep's minimum and the error bits, into the context's host scalars
+gm::MinOut cfl_out(gm_ctx* c) {
+  return gm::MinOut{&c->dscal->red, &c->hscal->dtmin, &c->dscal->err, &c->hscal->err, 0};
 }
 
 // the step of one precision: tstep (src/hydro_solver.f90:134-229)
@@ -528,9 +527,7 @@ void tstep_t(gm_ctx* c, double dt) {
   // the box), the next get_timestep's minimum is reduced in the same pass
   const bool fuse_cfl = fcd && !b.src && p.eta == 0.0 && !c->cool.kind && !c->cond.kind && !c->ubc_fn;
   if (fuse_cfl) {
-    hipLaunchKernelGGL(k_init_dtmin, dim3(1), dim3(1), 0, s, c->dscal);
-    timed(c, KC_BFIELD_CFL, [&] { gm::launch_bfield_cfl(s, b, dt, &c->dscal->dtmin, err, sh); });
-    (void)hipMemcpyAsync(c->hscal, c->dscal, sizeof(Scalars), hipMemcpyDeviceToHost, s);
+    timed(c, KC_BFIELD_CFL, [&] { gm::launch_bfield_cfl(s, b, dt, cfl_out(c), sh); });
     c->cfl_pending = true;
   } else if (fcd) {
     timed(c, KC_BFIELD, [&] { gm::launch_bfield(s, b, dt, 2, sh); });
@@ -555,7 +552,7 @@ void tstep_t(gm_ctx* c, double dt) {
 template <typename S>
 void cfl_t(gm_ctx* c) {
   const gm::Box<S> b = box_of<S>(c);
-  timed(c, KC_CFL, [&] { gm::launch_cfl(c->stream, b, &c->dscal->dtmin, &c->dscal->err, c->shape); });
+  timed(c, KC_CFL, [&] { gm::launch_cfl(c->stream, b, cfl_out(c), c->shape); });
 }
 
 int read_errors(gm_ctx* c) {
@@ -583,52 +580,66 @@ int read_errors(gm_ctx* c) {
 // ---------------------------------------------------------------------------
 constexpr size_t kScratchBytes = (size_t)256 << 20;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// the call's scalars, zero between calls
+__device__ Scalars scratch_scalars;
 
 constexpr int kMaxDevices = 64;
-void* g_scratch_ptr[kMaxDevices] = {nullptr};
+struct ScratchPtrs {
+  unsigned char* buf = nullptr;
+  Scalars* scal = nullptr;
+};
+ScratchPtrs g_scratch_ptr[kMaxDevices];
 std::mutex g_scratch_mu;
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// device bytes gm_tstep_noalloc needs for params (U*, W, E, scalars)
+// device bytes gm_tstep_noalloc needs for params (U*, W, E and 256 to spare)
 size_t noalloc_bytes(const gm_params* p) {
   const size_t ncell = (size_t)(p->nx + 4) * (p->ny + 4) * (p->nz + 4);
   const size_t es = p->precision == GM_PRECISION_MIXED ? 4 : 8, nq = (size_t)p->neq;
   return align256(ncell * nq * es) + align256(ncell * nq * sizeof(double)) + align256(ncell * 3 * es) +
-         align256(sizeof(Scalars));
+         256;
 }
 
-// address of this device's scratch array (the device is current)
-int scratch_of(int dev, unsigned char** out) {
+// addresses of this device's scratch array and scalars (the device is current)
+int scratch_of(int dev, ScratchPtrs* out) {
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_ptr[dev]) {
-    void* a = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&a, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !a) {
+  ScratchPtrs& g = g_scratch_ptr[dev];
+  if (!g.scal) {
+    void *a = nullptr, *b = nullptr;
+    hipError_t e = hipGetSymbolAddress(&a, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&b, HIP_SYMBOL(scratch_scalars));
+    if (e != hipSuccess || !a || !b) {
       (void)hipGetLastError();
       g_create_error = std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e);
       return GM_ERR_HIP;
     }
-    g_scratch_ptr[dev] = a;
+    g.buf = (unsigned char*)a;
+    g.scal = (Scalars*)b;
   }
-  *out = (unsigned char*)g_scratch_ptr[dev];
+  *out = g;
   return GM_OK;
 }
 
-__global__ void k_publish(const Scalars* sc, double* dtp, int32_t* err) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    if (dtp) *dtp = __longlong_as_double((long long)sc->dtmin);
-    if (err) *err = sc->err;
-  }
+// the scalars as a finished call leaves them, however the last one ended
+__global__ void k_idle_scalars(Scalars* s) {
+  s->red.slot[threadIdx.x].v = 0;
+  s->red.slot[threadIdx.x].count = 0;
+  if (threadIdx.x == 0) s->red.done = 0;
 }
 
 // tstep (src/hydro_solver.f90:134-229) with the add-ons a context adds
 // (user plugins, cooling, conduction) off: the kernels and order of
 // tstep_t, then get_timestep's minimum over the new state, as gm_cfl_dtp
-// computes it.  Scalars are set by kernels, not memsets, so a caller may
-// capture the launches in a graph.
+// computes it: the last kernel publishes it and the error bits, and clears
+// both for the next call.  (A call that raced another one may have left the
+// minimum's working space in disarray; the predictor's field update zeroes
+// it again.)  Kernels only, no memsets, so a caller may capture the launches
+// in a graph.
 template <typename S>
-void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, unsigned char* scr, double dt) {
+void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, const ScratchPtrs& sp, double dt, double* dtp_next,
+                     int32_t* err_out) {
+  unsigned char* scr = sp.buf;
   gm::Box<S> b;
   b.g.nx = p.nx; b.g.ny = p.ny; b.g.nz = p.nz;
   b.g.NX = p.nx + 4; b.g.NY = p.ny + 4; b.g.NZ = p.nz + 4;
@@ -652,14 +663,13 @@ void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, unsigned char* scr
   b.W = (double*)(scr + off);
   off += align256(ncell * nq * sizeof(double));
   b.E = (S*)(scr + off);
-  off += align256(ncell * 3 * sizeof(S));
-  Scalars* sc = (Scalars*)(scr + off);
+  Scalars* sc = sp.scal;
   b.dx = p.dx; b.dy = p.dy; b.dz = p.dz;
   b.slot = 0;
   b.src = p.eight_wave ? gm::SRC_EIGHT_WAVE : 0;
   b.srcin = (b.src != 0 && b.g.npas == 0) ? 1 : 0;
   b.usrc = nullptr;
-  const gm::Shape sh = {256, 16};
+  const gm::Shape sh = gm::column_shape(b.g);
   const int solver = p.riemann_solver, fcd = p.enable_flux_cd ? 1 : 0;
   int* err = &sc->err;
   const double dtm = dt / 2.0;  // hydro_solver.f90:152
@@ -673,20 +683,20 @@ void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, unsigned char* scr
       gm::launch_z(s, b, h, st, solver, fcd, err, sh);
     }
   };
-  hipLaunchKernelGGL(k_clear_err, dim3(1), dim3(1), 0, s, sc);
   stage(dtm, 1);
-  if (fcd) gm::launch_bfield(s, b, dtm, 1, sh);
+  if (fcd) gm::launch_bfield(s, b, dtm, 1, sh, &sc->red);
+  else hipLaunchKernelGGL(k_idle_scalars, dim3(1), dim3(gm::kMinSlots), 0, s, sc);
   if (b.src && !b.srcin) gm::launch_sources(s, b, dtm, 1, sh);
   stage(dt, 2);
-  hipLaunchKernelGGL(k_init_dtmin, dim3(1), dim3(1), 0, s, sc);
+  const gm::MinOut out{&sc->red, dtp_next, err, err_out, 1};
   const bool fuse_cfl = fcd && !b.src && p.eta == 0.0;
   if (fuse_cfl) {
-    gm::launch_bfield_cfl(s, b, dt, &sc->dtmin, err, sh);
+    gm::launch_bfield_cfl(s, b, dt, out, sh);
   } else {
     if (fcd) gm::launch_bfield(s, b, dt, 2, sh);
     if (b.src && !b.srcin) gm::launch_sources(s, b, dt, 2, sh);
     if (p.eta != 0.0) gm::launch_viscous(s, b, p.eta);
-    gm::launch_cfl(s, b, &sc->dtmin, err, sh);
+    gm::launch_cfl(s, b, out, sh);
   }
 }
 
@@ -717,12 +727,13 @@ int gm_create(const gm_params* params, gm_ctx** out) {
   c->ph.eos = GM_EOS_ADIABATIC;
   c->ph.tempsc = 1.0;
   stage_policy(params->precision, g, c->slab_kchunk);
+  c->shape = gm::column_shape(g);
   // GUACHO_AMD_COLUMN_SHAPE="block,kchunk" overrides the column kernels'
-  // tile width (64, 128 or 256 threads) and z-pencil length
+  // tile width (64, 128 or 256 threads) and z-pencil lengths
   if (const char* e = std::getenv("GUACHO_AMD_COLUMN_SHAPE")) {
     int bl = 0, kc = 0;
     if (std::sscanf(e, "%d,%d", &bl, &kc) == 2 && (bl == 64 || bl == 128 || bl == 256) && kc >= 1 && kc <= 4096)
-      c->shape = {bl, kc, 0};
+      c->shape = gm::Shape{bl, kc, kc, 0, 0};
   }
 
   auto bail = [&](int code) {
@@ -748,12 +759,13 @@ int gm_create(const gm_params* params, gm_ctx** out) {
     c->bytes += (int64_t)a.n;
   }
   if ((rc = hip_check(c, hipMalloc((void**)&c->dscal, sizeof(Scalars)), "hipMalloc")) != GM_OK) return bail(rc);
-  if ((rc = hip_check(c, hipHostMalloc((void**)&c->hscal, sizeof(Scalars), hipHostMallocDefault),
+  if ((rc = hip_check(c, hipHostMalloc((void**)&c->hscal, sizeof(HostScalars), hipHostMallocDefault),
                       "hipHostMalloc")) != GM_OK)
     return bail(rc);
   // zero everything once so no kernel ever reads uninitialised memory
   for (auto& a : allocs) (void)hipMemsetAsync(*a.p, 0, a.n, c->stream);
   (void)hipMemsetAsync(c->dscal, 0, sizeof(Scalars), c->stream);
+  *c->hscal = HostScalars{};
   if ((rc = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize")) != GM_OK) return bail(rc);
   *out = c;
   return GM_OK;
@@ -861,16 +873,13 @@ int gm_cfl_dtp(gm_ctx* c, double* dtp) {
   int rc = set_device(c);
   if (rc) return rc;
   if (!c->cfl_ready) {
-    hipLaunchKernelGGL(k_init_dtmin, dim3(1), dim3(1), 0, c->stream, c->dscal);
     if (c->esize == 8) cfl_t<double>(c);
     else cfl_t<float>(c);
     GM_HIP(c, hipGetLastError());
-    GM_HIP(c, hipMemcpyAsync(c->hscal, c->dscal, sizeof(Scalars), hipMemcpyDeviceToHost, c->stream));
   }
   c->cfl_ready = false;
   GM_HIP(c, hipStreamSynchronize(c->stream));
-  const unsigned long long bits = c->hscal->dtmin;
-  std::memcpy(dtp, &bits, sizeof(double));
+  *dtp = c->hscal->dtmin;
   if (c->hscal->err) return read_errors(c);
   return GM_OK;
 }
@@ -1105,13 +1114,11 @@ int gm_tstep_noalloc(const gm_params* params, void* u, double dt, void* stream, 
   if (!std::isfinite(dt)) return fail(nullptr, GM_ERR_ARG, "dt is not finite");
   if (params->device < 0 || params->device >= kMaxDevices) return fail(nullptr, GM_ERR_ARG, "device out of range");
   if ((rc = hip_check(nullptr, hipSetDevice(params->device), "hipSetDevice")) != GM_OK) return rc;
-  unsigned char* scr = nullptr;
-  if ((rc = scratch_of(params->device, &scr)) != GM_OK) return rc;
+  ScratchPtrs sp;
+  if ((rc = scratch_of(params->device, &sp)) != GM_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (params->precision == GM_PRECISION_MIXED) noalloc_tstep_t<float>(s, *params, (float*)u, scr, dt);
-  else noalloc_tstep_t<double>(s, *params, (double*)u, scr, dt);
-  const size_t off = noalloc_bytes(params) - align256(sizeof(Scalars));
-  if (dtp_next || err) hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, s, (const Scalars*)(scr + off), dtp_next, err);
+  if (params->precision == GM_PRECISION_MIXED) noalloc_tstep_t<float>(s, *params, (float*)u, sp, dt, dtp_next, err);
+  else noalloc_tstep_t<double>(s, *params, (double*)u, sp, dt, dtp_next, err);
   return hip_check(nullptr, hipGetLastError(), "kernel launch");
 }
 

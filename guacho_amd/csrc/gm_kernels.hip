@@ -1711,8 +1711,50 @@ __device__ __forceinline__ TcCell tc_cell(const Box<S>& b, const Conduction& tc,
   return r;
 }
 
+// The workgroup's minimum m (thread 0's) into a MinRed; see there.  Wave 0
+// of every workgroup calls it.  Relaxed atomics, each waited for before the
+// next one that counts on it: the order they need without the cache
+// write-back of a release.
+__device__ __forceinline__ void min_publish(double m, const MinOut& o) {
+  const int lane = (int)threadIdx.x;
+  const unsigned nb = gridDim.x, s = blockIdx.x % kMinSlots;
+  const unsigned ns = nb < (unsigned)kMinSlots ? nb : (unsigned)kMinSlots;
+  MinRed* r = o.red;
+  int last = 0;
+  if (lane == 0) {
+    (void)__hip_atomic_fetch_max(&r->slot[s].v, ~(unsigned long long)__double_as_longlong(m), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned mine = (nb - s + kMinSlots - 1) / kMinSlots;  // workgroups of this slot
+    if (__hip_atomic_fetch_add(&r->slot[s].count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == mine)
+      last = __hip_atomic_fetch_add(&r->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == ns;
+  }
+  if (!__builtin_amdgcn_readfirstlane(last)) return;
+  unsigned long long v = 0;
+  if (lane < (int)ns) {
+    v = __hip_atomic_load(&r->slot[lane].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&r->slot[lane].v, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&r->slot[lane].count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long w = __shfl_xor(v, off, 64);
+    v = w > v ? w : v;
+  }
+  if (lane == 0) {
+    __hip_atomic_store(&r->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (o.min)
+      __hip_atomic_store((unsigned long long*)o.min, ~v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (o.err_out) {
+      const int e = __hip_atomic_load(o.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(o.err_out, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (o.clear_err) __hip_atomic_store(o.err, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
 template <typename S>
-__global__ void __launch_bounds__(256) k_tc_dtmin(Box<S> b, Conduction tc, unsigned long long* out) {
+__global__ void __launch_bounds__(256) k_tc_dtmin(Box<S> b, Conduction tc, MinOut out) {
   __shared__ double red[4];
   const Geom& g = b.g;
   const long long n = (long long)g.nx * g.ny * g.nz;
@@ -1729,10 +1771,10 @@ __global__ void __launch_bounds__(256) k_tc_dtmin(Box<S> b, Conduction tc, unsig
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) red[wid] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (wid == 0) {
     double m = red[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = tc_min(m, red[w]);
-    atomicMin(out, (unsigned long long)__double_as_longlong(m));
+    min_publish(m, out);
   }
 }
 
@@ -1917,32 +1959,44 @@ __device__ __forceinline__ double cfl_cell(const Phys& ph, double dx, double dy,
   return dtp;
 }
 
-// the workgroup's minimum into *dtmin (positive doubles order as their bit
-// patterns); a non-finite conserved value sets bit 2 of *err.  Every thread
-// of the workgroup (at most 256) calls it.
-__device__ __forceinline__ void cfl_reduce(double dtp, bool bad, unsigned long long* __restrict__ dtmin,
-                                           int* __restrict__ err) {
+// the workgroup's minimum, valid in wave 0; a non-finite conserved value
+// sets bit 2 of *err.  Every thread of the workgroup (at most 256) calls it.
+__device__ __forceinline__ double cfl_block_min(double dtp, bool bad, int* __restrict__ err) {
   __shared__ double red[4];
   if (__any(bad)) {
     if ((threadIdx.x & 63) == 0) atomicOr(err, 2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // before the workgroup counts itself done
   }
   dtp = wave_min(dtp);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) red[wid] = dtp;
   __syncthreads();
+  double m = red[0];
+  for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = dmin(m, red[w]);
+  return m;
+}
+
+// ... published by the launch (one box)
+__device__ __forceinline__ void cfl_reduce(double dtp, bool bad, const MinOut& out) {
+  const double m = cfl_block_min(dtp, bad, out.err);
+  if (threadIdx.x < 64) min_publish(m, out);
+}
+
+// ... or into a batch's clock (positive doubles order as their bit
+// patterns): an atomic only where it lowers the value, as atomics on one
+// address are serial
+__device__ __forceinline__ void cfl_reduce(double dtp, bool bad, unsigned long long* __restrict__ dtmin,
+                                           int* __restrict__ err) {
+  const double m = cfl_block_min(dtp, bad, err);
   if (threadIdx.x == 0) {
-    double m = red[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++) m = dmin(m, red[w]);
-    atomicMin(dtmin, (unsigned long long)__double_as_longlong(m));
+    const unsigned long long v = (unsigned long long)__double_as_longlong(m);
+    if (v < __hip_atomic_load(dtmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(dtmin, v);
   }
 }
 
 template <typename S, int NQ = 8>
-__device__ __forceinline__ void cfl_body(const Box<S>& b, unsigned lb, int kchunk,
-                                         unsigned long long* __restrict__ dtmin, int* __restrict__ err) {
+__device__ __forceinline__ void cfl_body(const Box<S>& b, unsigned lb, int kchunk, double& dtp, bool& bad) {
   const Geom& g = b.g;
-  double dtp = 1e30;
-  bool bad = false;
   int t, kc;
   if (tile_item(lb, tiles_of((unsigned)(g.nx * g.ny)), (unsigned)(g.nx * g.ny), t, kc)) {
     const int i = t % g.nx + 1, j = t / g.nx + 1;
@@ -1959,7 +2013,6 @@ __device__ __forceinline__ void cfl_body(const Box<S>& b, unsigned lb, int kchun
       dtp = cfl_cell<NQ, S>(b.ph, b.dx, b.dy, b.dz, u, dtp, b.pc ? b.pc + c : nullptr);
     }
   }
-  cfl_reduce(dtp, bad, dtmin, err);
 }
 
 // ---------------------------------------------------------------------------
@@ -1996,7 +2049,12 @@ k_slab(Box<S> b, double dt, int kchunk, int* err) {
 }
 
 template <typename S>
-__global__ void __launch_bounds__(256) k_bfield(Box<S> b, double dt, int stage, int kchunk) {
+__global__ void __launch_bounds__(256) k_bfield(Box<S> b, double dt, int stage, int kchunk, MinRed* idle) {
+  if (idle && blockIdx.x == 0 && threadIdx.x < kMinSlots) {
+    idle->slot[threadIdx.x].v = 0;
+    idle->slot[threadIdx.x].count = 0;
+    if (threadIdx.x == 0) idle->done = 0;
+  }
   // the predictor's field update runs its tiles in the reverse of the slab
   // kernel's order (E written last is read first, from the memory-side
   // cache); the corrector's, after the reversed z kernel, runs forward
@@ -2009,17 +2067,27 @@ __global__ void __launch_bounds__(256) k_bfield(Box<S> b, double dt, int stage, 
 // nothing after the field update changes U's interior the reduction needs
 // no pass of its own over U
 template <typename S, int NQ>
-__global__ void __launch_bounds__(256) k_bfield_cfl(Box<S> b, double dt, int kchunk, unsigned long long* dtmin,
-                                                    int* err) {
+__global__ void __launch_bounds__(256) k_bfield_cfl(Box<S> b, double dt, int kchunk, MinOut out) {
   double dtp = 1e30;
   bool bad = false;
   bfield_body<S, 1, NQ>(b, xcd_logical_block(), dt, 2, kchunk, &dtp, &bad);
-  cfl_reduce(dtp, bad, dtmin, err);
+  cfl_reduce(dtp, bad, out);
 }
 
 template <typename S, int NQ>
-__global__ void __launch_bounds__(256) k_cfl(Box<S> b, int kchunk, unsigned long long* dtmin, int* err) {
-  cfl_body<S, NQ>(b, xcd_logical_block(), kchunk, dtmin, err);
+__global__ void __launch_bounds__(256) k_cfl(Box<S> b, int kchunk, MinOut out) {
+  double dtp = 1e30;
+  bool bad = false;
+  cfl_body<S, NQ>(b, xcd_logical_block(), kchunk, dtp, bad);
+  cfl_reduce(dtp, bad, out);
+}
+
+template <typename S, int NQ>
+__global__ void __launch_bounds__(256) k_cfl_clock(Box<S> b, int kchunk, unsigned long long* dtmin, int* err) {
+  double dtp = 1e30;
+  bool bad = false;
+  cfl_body<S, NQ>(b, xcd_logical_block(), kchunk, dtp, bad);
+  cfl_reduce(dtp, bad, dtmin, err);
 }
 
 template <typename S>
@@ -2141,7 +2209,10 @@ __global__ void __launch_bounds__(256) kb_cfl(const Box<S>* __restrict__ boxes, 
   int bx;
   unsigned lb;
   batch_locate(prefix, nbox, xcd_logical_block(), bx, lb);
-  cfl_body<S, NQ>(boxes[bx], lb, kchunk, &clk[boxes[bx].slot].dtmin, err);
+  double dtp = 1e30;
+  bool bad = false;
+  cfl_body<S, NQ>(boxes[bx], lb, kchunk, dtp, bad);
+  cfl_reduce(dtp, bad, &clk[boxes[bx].slot].dtmin, err);
 }
 
 
@@ -2307,6 +2378,7 @@ unsigned box_tiles(const Geom& g, int kclass, const Shape& sh) {
   switch (kclass) {
     case KC_XY: return ceil_div(g.nx, TX) * ceil_div(g.ny, TY) * (unsigned)g.nz;
     case KC_COL: return ceil_div((long long)g.nx * g.ny, sh.block) * ceil_div(g.nz, sh.kchunk);
+    case KC_FIELD: return ceil_div((long long)g.nx * g.ny, sh.block) * ceil_div(g.nz, sh.fchunk);
     case KC_SLAB: return sh.slab > 0 ? slab_tiles(g, sh.slab) : 0u;
   }
   return 0;
@@ -2330,7 +2402,7 @@ unsigned box_tiles(const Geom& g, int kclass, const Shape& sh) {
 
 template <typename S>
 void launch_xy(hipStream_t s, const Box<S>& b, double dt, int stage, int solver, int flux_cd, int* err) {
-  const unsigned n = box_tiles(b.g, KC_XY, Shape{XY_THREADS, 1});
+  const unsigned n = box_tiles(b.g, KC_XY, Shape{});
 #define GM_CALL(SV, O, F)                                                                                  \
   {                                                                                                        \
     if (b.g.npas == 0) hipLaunchKernelGGL((k_xy<SV, O, F, S, 0>), dim3(n), dim3(XY_THREADS), 0, s, b, dt, err); \
@@ -2415,28 +2487,48 @@ void launch_slab(hipStream_t s, const Box<S>& b, double dt, int stage, int solve
 }
 
 template <typename S>
-void launch_bfield(hipStream_t s, const Box<S>& b, double dt, int stage, const Shape& sh) {
-  hipLaunchKernelGGL(k_bfield<S>, dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, dt, stage, sh.kchunk);
+void launch_bfield(hipStream_t s, const Box<S>& b, double dt, int stage, const Shape& sh, MinRed* idle) {
+  hipLaunchKernelGGL(k_bfield<S>, dim3(box_tiles(b.g, KC_FIELD, sh)), dim3(sh.block), 0, s, b, dt, stage, sh.fchunk, idle);
 }
 
 template <typename S>
-void launch_bfield_cfl(hipStream_t s, const Box<S>& b, double dt, unsigned long long* dtmin, int* err,
-                       const Shape& sh) {
-  if (b.g.npas == 0)
-    hipLaunchKernelGGL((k_bfield_cfl<S, 8>), dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, dt,
-                       sh.kchunk, dtmin, err);
-  else
-    hipLaunchKernelGGL((k_bfield_cfl<S, 10>), dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, dt,
-                       sh.kchunk, dtmin, err);
+void launch_bfield_cfl(hipStream_t s, const Box<S>& b, double dt, const MinOut& out, const Shape& sh) {
+  const dim3 n(box_tiles(b.g, KC_FIELD, sh));
+  if (b.g.npas == 0) hipLaunchKernelGGL((k_bfield_cfl<S, 8>), n, dim3(sh.block), 0, s, b, dt, sh.fchunk, out);
+  else hipLaunchKernelGGL((k_bfield_cfl<S, 10>), n, dim3(sh.block), 0, s, b, dt, sh.fchunk, out);
 }
 
 template <typename S>
-void launch_cfl(hipStream_t s, const Box<S>& b, unsigned long long* dtmin, int* err, const Shape& sh) {
-  if (b.g.npas == 0)
-    hipLaunchKernelGGL((k_cfl<S, 8>), dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, sh.kchunk, dtmin, err);
-  else  // EOS_H_RATE reads the first passive scalar
-    hipLaunchKernelGGL((k_cfl<S, 10>), dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, sh.kchunk, dtmin, err);
+void launch_cfl(hipStream_t s, const Box<S>& b, const MinOut& out, const Shape& sh) {
+  const dim3 n(box_tiles(b.g, KC_FIELD, sh));
+  if (b.g.npas == 0) hipLaunchKernelGGL((k_cfl<S, 8>), n, dim3(sh.block), 0, s, b, sh.fchunk, out);
+  else hipLaunchKernelGGL((k_cfl<S, 10>), n, dim3(sh.block), 0, s, b, sh.fchunk, out);  // EOS_H_RATE reads the first passive scalar
 }
+
+template <typename S>
+void launch_cfl_clock(hipStream_t s, const Box<S>& b, unsigned long long* dtmin, int* err, const Shape& sh) {
+  const dim3 n(box_tiles(b.g, KC_FIELD, sh));
+  if (b.g.npas == 0) hipLaunchKernelGGL((k_cfl_clock<S, 8>), n, dim3(sh.block), 0, s, b, sh.fchunk, dtmin, err);
+  else hipLaunchKernelGGL((k_cfl_clock<S, 10>), n, dim3(sh.block), 0, s, b, sh.fchunk, dtmin, err);
+}
+
+#if GM_PART(1)
+// Pencils of 16 cells everywhere left small grids with a serial march on a
+// few CUs.  A z-face pencil pays a window warm-up of about three cells and
+// its kernel holds two workgroups per CU in FP64, so it shortens to one round
+// of the 512 resident workgroups; a field update or CFL pencil carries two
+// values at most, so it shortens to 1024 workgroups (half of what the GPU
+// holds).  From 128^3 (z) and 256x256x64 (field) on both are 16.  Per launch,
+// 16 cells against this rule, FP64 (mixed): z corrector 96^3 48.8 us against
+// 43.3 (39.8, 27.8), 150x70x45 44.4 against 30.1 (36.9, 19.9); field update
+// with the CFL minimum 64^3 34.6 against 13.8 (35.9, 12.7), 128x128x4 15.2
+// against 10.4, 113^3 51.7 against 41.9; field update 64^3 16.0 against 9.2.
+Shape column_shape(const Geom& g) {
+  const long long work = (long long)ceil_div((long long)g.nx * g.ny, 256) * g.nz;  // tiles x planes
+  auto clamp = [](long long v, int lo, int hi) { return (int)(v < lo ? lo : v > hi ? hi : v); };
+  return Shape{256, clamp((work + 511) / 512, 4, 16), clamp((work + 1023) / 1024, 1, 16), 0, 0};
+}
+#endif
 
 template <typename S>
 void launch_viscous(hipStream_t s, const Box<S>& b, double eta) {
@@ -2454,7 +2546,7 @@ void launch_cooling(hipStream_t s, const Box<S>& b, const Cooling& cl, double dt
 }
 
 template <typename S>
-void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, unsigned long long* out) {
+void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, const MinOut& out) {
   const long long n = (long long)b.g.nx * b.g.ny * b.g.nz;
   hipLaunchKernelGGL(k_tc_dtmin<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, tc, out);
 }
@@ -2486,20 +2578,20 @@ void launch_tc_substep(hipStream_t s, const Box<S>& b, const Conduction& tc, dou
 
 template <typename S>
 void launch_sources(hipStream_t s, const Box<S>& b, double dt, int stage, const Shape& sh) {
-  hipLaunchKernelGGL(k_sources<S>, dim3(box_tiles(b.g, KC_COL, sh)), dim3(sh.block), 0, s, b, dt, stage, sh.kchunk);
+  hipLaunchKernelGGL(k_sources<S>, dim3(box_tiles(b.g, KC_FIELD, sh)), dim3(sh.block), 0, s, b, dt, stage, sh.fchunk);
 }
 
 template <typename S>
 void launch_sources_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefix, int nbox, unsigned tiles,
                           const BoxClock* clk, int stage, const Shape& sh) {
-  hipLaunchKernelGGL(kb_sources<S>, dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, stage, sh.kchunk);
+  hipLaunchKernelGGL(kb_sources<S>, dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, stage, sh.fchunk);
 }
 
 template <typename S>
 void launch_viscous_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefix, int nbox, unsigned tiles,
                           const BoxClock* clk, const Shape& sh) {
-  hipLaunchKernelGGL((kb_viscous<S, false>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.kchunk);
-  hipLaunchKernelGGL((kb_viscous<S, true>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.kchunk);
+  hipLaunchKernelGGL((kb_viscous<S, false>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.fchunk);
+  hipLaunchKernelGGL((kb_viscous<S, true>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.fchunk);
 }
 
 template <typename S>
@@ -2546,22 +2638,22 @@ void launch_slab_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefi
 template <typename S>
 void launch_bfield_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefix, int nbox, unsigned tiles,
                          const BoxClock* clk, int stage, const Shape& sh) {
-  hipLaunchKernelGGL(kb_bfield<S>, dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, stage, sh.kchunk);
+  hipLaunchKernelGGL(kb_bfield<S>, dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, stage, sh.fchunk);
 }
 
 template <typename S>
 void launch_bfield_cfl_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefix, int nbox, unsigned tiles,
                              BoxClock* clk, int* err, const Shape& sh, int npas) {
   // as launch_bfield_cfl: with passive scalars every variable through NQ = 10
-  if (npas == 0) hipLaunchKernelGGL((kb_bfield_cfl<S, 8>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.kchunk, err);
-  else hipLaunchKernelGGL((kb_bfield_cfl<S, 10>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.kchunk, err);
+  if (npas == 0) hipLaunchKernelGGL((kb_bfield_cfl<S, 8>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.fchunk, err);
+  else hipLaunchKernelGGL((kb_bfield_cfl<S, 10>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, clk, sh.fchunk, err);
 }
 
 template <typename S>
 void launch_cfl_batch(hipStream_t s, const Box<S>* boxes, const unsigned* prefix, int nbox, unsigned tiles,
                       BoxClock* clk, int* err, const Shape& sh, int npas) {
-  if (npas == 0) hipLaunchKernelGGL((kb_cfl<S, 8>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, sh.kchunk, clk, err);
-  else hipLaunchKernelGGL((kb_cfl<S, 10>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, sh.kchunk, clk, err);
+  if (npas == 0) hipLaunchKernelGGL((kb_cfl<S, 8>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, sh.fchunk, clk, err);
+  else hipLaunchKernelGGL((kb_cfl<S, 10>), dim3(tiles), dim3(sh.block), 0, s, boxes, prefix, nbox, sh.fchunk, clk, err);
 }
 
 #if GM_PART(1)
@@ -2616,13 +2708,14 @@ void launch_divb(hipStream_t s, const Geom& g, const S* U, double dx, double dy,
 #define GM_INST_SLAB(S)                                                                                          \
   template void launch_slab<S>(hipStream_t, const Box<S>&, double, int, int, int, int*, int);
 #define GM_INST_REST(S)                                                                                          \
-  template void launch_bfield<S>(hipStream_t, const Box<S>&, double, int, const Shape&);                          \
-  template void launch_cfl<S>(hipStream_t, const Box<S>&, unsigned long long*, int*, const Shape&);               \
-  template void launch_bfield_cfl<S>(hipStream_t, const Box<S>&, double, unsigned long long*, int*, const Shape&); \
+  template void launch_bfield<S>(hipStream_t, const Box<S>&, double, int, const Shape&, MinRed*);                 \
+  template void launch_cfl<S>(hipStream_t, const Box<S>&, const MinOut&, const Shape&);                           \
+  template void launch_cfl_clock<S>(hipStream_t, const Box<S>&, unsigned long long*, int*, const Shape&);         \
+  template void launch_bfield_cfl<S>(hipStream_t, const Box<S>&, double, const MinOut&, const Shape&);            \
   template void launch_sources<S>(hipStream_t, const Box<S>&, double, int, const Shape&);                         \
   template void launch_cooling<S>(hipStream_t, const Box<S>&, const Cooling&, double);                            \
   template void launch_viscous<S>(hipStream_t, const Box<S>&, double);                                            \
-  template void launch_tc_dtmin<S>(hipStream_t, const Box<S>&, const Conduction&, unsigned long long*);           \
+  template void launch_tc_dtmin<S>(hipStream_t, const Box<S>&, const Conduction&, const MinOut&);                 \
   template void launch_tc_substep<S>(hipStream_t, const Box<S>&, const Conduction&, double);                      \
   template void launch_ghost<S>(hipStream_t, const Geom&, S*, int, int, int, int);                               \
   template void launch_aos_to_soa<S>(hipStream_t, long long, const double*, S*, int);                             \

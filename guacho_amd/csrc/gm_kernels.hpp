@@ -85,23 +85,51 @@ struct BoxClock {
   int pad;
 };
 
-// Launch shape of the column-marching kernels (z faces, field update, CFL):
-// threads per tile (64, 128 or 256) and z-pencil length.  The xy-face
-// kernel has a fixed 32 x 16 plane tile.
+// Launch shape of the column-marching kernels: threads per tile (64, 128 or
+// 256), the z-face kernel's pencil length and that of the field update, CFL
+// and source kernels.  The xy-face kernel has a fixed 32 x 16 plane tile.
 struct Shape {
   int block;
   int kchunk;
+  int fchunk;
   int slab;        // planes per slab of the 2.5-D stage kernel; 0: the two-kernel stage
   int slab_both;   // batches: 1 when the corrector runs as the slab kernel too
+};
+
+// the column kernels' shape for one grid
+Shape column_shape(const Geom& g);
+
+// Minimum over all workgroups of a launch, published by the launch itself.
+// Atomics on one address are serial here at 11.5 ns each (4096 workgroups:
+// 47 us), so workgroup b reduces into slot b % kMinSlots; the last workgroup
+// of a slot counts the slot done, the last slot's workgroup writes the
+// result and leaves every field zero, as it found it: a launch needs no
+// reset before it and no copy behind it: two launches fewer a step, 128x128x4
+// FP64 75 -> 67 us a step together with the shorter pencils of column_shape.
+constexpr int kMinSlots = 64;
+struct MinRed {
+  struct alignas(64) Slot {
+    unsigned long long v;  // complement of the minimum's bits (a positive double), a maximum over the slot's workgroups
+    unsigned count;        // workgroups that have added theirs
+  } slot[kMinSlots];
+  unsigned done;           // slots complete
+};
+struct MinOut {
+  MinRed* red;
+  double* min;      // the result: device memory or pinned host memory
+  int* err;         // the kernels' error bits ...
+  int* err_out;     // ... copied here when not null
+  int clear_err;    // and cleared after the copy
 };
 
 // Validates a subdomain configuration; GM_OK or a GM_ERR_* code with msg.
 int check_params(const gm_params* p, std::string& msg);
 
 // Tile classes of one step, for per-class tile tables: 32 x 16 plane tiles
-// of the xy-face kernel, column pencils of the z-face, field-update and CFL
-// kernels, and 32 x 8 column tiles of the slab kernel (Shape::slab planes).
-enum KClass { KC_XY = 0, KC_COL, KC_SLAB, KC_COUNT };
+// of the xy-face kernel, column pencils of the z-face kernel and of the
+// field-update, CFL and source kernels, and 32 x 8 column tiles of the slab
+// kernel (Shape::slab planes).
+enum KClass { KC_XY = 0, KC_COL, KC_FIELD, KC_SLAB, KC_COUNT };
 
 // Tiles (workgroups) one box needs for a kernel class under a shape.
 unsigned box_tiles(const Geom& g, int kclass, const Shape& sh);
@@ -127,15 +155,20 @@ void launch_slab(hipStream_t s, const Box<S>& b, double dt, int stage, int solve
 // default slab length for a grid, and the workgroups of a slab launch
 int slab_kchunk(const Geom& g, int resident);
 unsigned slab_tiles(const Geom& g, int kchunk);
+// `idle`: a MinRed to zero on the way (null: none), for a caller that does
+// not know how the last launch over it ended
 template <typename S>
-void launch_bfield(hipStream_t s, const Box<S>& b, double dt, int stage, const Shape& sh);
+void launch_bfield(hipStream_t s, const Box<S>& b, double dt, int stage, const Shape& sh, MinRed* idle = nullptr);
+// get_timestep's minimum over the state, published through `out`
 template <typename S>
-void launch_cfl(hipStream_t s, const Box<S>& b, unsigned long long* dtmin, int* err, const Shape& sh);
+void launch_cfl(hipStream_t s, const Box<S>& b, const MinOut& out, const Shape& sh);
+// the same into *dtmin, which must hold 1e30 beforehand (a batch's clock)
+template <typename S>
+void launch_cfl_clock(hipStream_t s, const Box<S>& b, unsigned long long* dtmin, int* err, const Shape& sh);
 // the corrector's field update (stage 2 of launch_bfield) plus launch_cfl's
-// reduction over the updated state; *dtmin must hold 1e30 beforehand
+// reduction over the updated state
 template <typename S>
-void launch_bfield_cfl(hipStream_t s, const Box<S>& b, double dt, unsigned long long* dtmin, int* err,
-                       const Shape& sh);
+void launch_bfield_cfl(hipStream_t s, const Box<S>& b, double dt, const MinOut& out, const Shape& sh);
 // cooling pass on U^{n+1} (src/hydro_solver.f90:206-210) with the step's dt
 // viscous_copy with eta != 0 (W as scratch), after the corrector
 template <typename S>
@@ -149,10 +182,10 @@ struct Conduction {
   int kind, sat;
   double tempsc, rsc, rhosc, mu, psc, tsc, vsc2, bsc;
 };
-// min over interior cells of rho / Ksp(T), as the bit pattern of a positive
-// double atomically reduced into *out (get_dt_cond's loop, :78-110)
+// min over interior cells of rho / Ksp(T) (get_dt_cond's loop, :78-110),
+// published through `out`
 template <typename S>
-void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, unsigned long long* out);
+void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, const MinOut& out);
 // one sub-step: heat fluxes of cells 0..n (into W), the E update of the
 // interior with dts, thermal_bounds on E
 template <typename S>
