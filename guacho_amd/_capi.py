@@ -198,13 +198,13 @@ class Subdomain:
         self._check(self.L.gm_upload_u(self.h, u))
 
     def download_u(self) -> np.ndarray:
-        u = np.zeros(self.shape, dtype=np.float64, order="F")
+        u = np.empty(self.shape, dtype=np.float64, order="F")
         self._check(self.L.gm_download_u(self.h, u))
         return u
 
     def download_primit(self, with_temp: bool = False):
-        p = np.zeros(self.shape, dtype=np.float64, order="F")
-        t = np.zeros(self.shape[1:], dtype=np.float64, order="F") if with_temp else None
+        p = np.empty(self.shape, dtype=np.float64, order="F")
+        t = np.empty(self.shape[1:], dtype=np.float64, order="F") if with_temp else None
         self._check(self.L.gm_download_primit(self.h, p, t.ctypes.data if t is not None else None))
         return (p, t) if with_temp else p
 
@@ -224,7 +224,7 @@ class Subdomain:
 
     def divb(self) -> np.ndarray:
         p = self.params
-        d = np.zeros((p.nx, p.ny, p.nz), dtype=np.float64, order="F")
+        d = np.empty((p.nx, p.ny, p.nz), dtype=np.float64, order="F")
         self._check(self.L.gm_download_divb(self.h, d))
         return d
 
@@ -373,7 +373,7 @@ class Batch:
         return t.value, n.value, bool(d.value)
 
     def download_u(self, box: int) -> np.ndarray:
-        u = np.zeros(self.shapes[box], dtype=np.float64, order="F")
+        u = np.empty(self.shapes[box], dtype=np.float64, order="F")
         self._check(self.L.gm_batch_download_u(self.h, box, u))
         return u
 

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "gm_kernels.hpp"
+#include "gm_xfer.hpp"
 #include "guacho_amd.h"
 
 namespace {
@@ -33,18 +34,26 @@ unsigned long long gm_bits_of(double x) {
   return u;
 }
 
+// One allocation of the batch; a box's buffers lie in one.
+struct Block {
+  char* p = nullptr;
+  int64_t bytes = 0;
+};
+
 struct Slot {
   bool used = false;
   gm_params p{};
+  Block block;
   void* U = nullptr;
   void* Us = nullptr;
   void* W = nullptr;  // stage partials, 8 doubles per cell; also upload/download staging
   void* E = nullptr;
-  int64_t bytes = 0;
+  int64_t bytes = 0;  // counted against the budget
   gm::BoxClock clock{};  // host copy as of the last sync
 };
 
 constexpr int kMaxBoxes = 4096;
+constexpr int64_t kSpareMax = (int64_t)1 << 30;
 
 }  // namespace
 
@@ -69,7 +78,14 @@ struct gm_batch {
   bool in_flight = false;
   std::vector<int> launched;
   hipEvent_t ev_launch = nullptr;
-  std::vector<void*> zombies;
+  std::vector<Block> zombies;
+  // Blocks of released boxes, for boxes to come: an allocation and its
+  // release cost more than a small box's steps.  At most kSpareMax bytes and
+  // within the budget together with the boxes (a reused block may be up to
+  // an eighth larger than its box); they go with the batch.
+  std::vector<Block> spare;
+  int64_t spare_bytes = 0;
+  int64_t held = 0;  // bytes of all blocks
   bool any_sources = false;        // some active box has 8-wave source terms
   bool any_viscous = false;        // some active box has artificial viscosity
   int neq = 8;                     // variables of every box: 8 + its passive scalars (the first box sets it)
@@ -157,11 +173,51 @@ gm::Box<S> box_view(const Slot& s, int slot) {
   return b;
 }
 
-void free_slot(Slot& s) {
-  void* bufs[] = {s.U, s.Us, s.W, s.E};
-  for (void* p : bufs)
-    if (p) (void)hipFree(p);
-  s = Slot();
+void drop_block(gm_batch* b, const Block& k) {
+  if (k.p) (void)hipFree(k.p);
+  b->held -= k.bytes;
+}
+
+Block take_spare(gm_batch* b, size_t i) {
+  const Block k = b->spare[i];
+  b->spare.erase(b->spare.begin() + (long)i);
+  b->spare_bytes -= k.bytes;
+  return k;
+}
+
+// The block of a box that no launch in flight steps.
+void give_block(gm_batch* b, const Block& k) {
+  if (b->spare_bytes + k.bytes <= kSpareMax) {
+    b->spare.push_back(k);
+    b->spare_bytes += k.bytes;
+  } else if (b->in_flight) {
+    b->zombies.push_back(k);  // freeing could wait for the launches in flight
+  } else {
+    drop_block(b, k);
+  }
+}
+
+// A block of at least `need` bytes: the best fitting spare one, else a new
+// one, for which spare blocks make room.  No block (p null): out of memory.
+Block take_block(gm_batch* b, int64_t need) {
+  size_t best = b->spare.size();
+  for (size_t i = 0; i < b->spare.size(); i++)
+    if (b->spare[i].bytes >= need && b->spare[i].bytes <= need + need / 8 &&
+        (best == b->spare.size() || b->spare[i].bytes < b->spare[best].bytes))
+      best = i;
+  if (best < b->spare.size()) return take_spare(b, best);
+  while (!b->spare.empty() && b->held + need > b->budget) drop_block(b, take_spare(b, 0));
+  Block k;
+  void* p = nullptr;
+  while (hipMalloc(&p, (size_t)need) != hipSuccess) {
+    (void)hipGetLastError();
+    if (b->spare.empty()) return k;
+    drop_block(b, take_spare(b, 0));
+  }
+  k.p = (char*)p;
+  k.bytes = need;
+  b->held += need;
+  return k;
 }
 
 void drop_graph(gm_batch* b) {
@@ -340,7 +396,7 @@ int autotune(gm_batch* b) {
 }
 
 void free_zombies(gm_batch* b) {
-  for (void* p : b->zombies) (void)hipFree(p);
+  for (const Block& k : b->zombies) drop_block(b, k);
   b->zombies.clear();
 }
 
@@ -419,6 +475,7 @@ int gm_batch_create(const gm_batch_params* bp, gm_batch** out) {
     return bfail(nullptr, GM_ERR_CONFIG, "steps_per_launch must be in 1..1000");
   if (bp->reserved != 0 || bp->memory_budget < 0) return bfail(nullptr, GM_ERR_CONFIG, "bad reserved / budget field");
   gm_batch* b = new gm_batch();
+  gm::xfer_retain();  // released with the batch
   b->bp = *bp;
   // stage kernels before (or without) autotuning: the two-kernel stage, or
   // GUACHO_AMD_BATCH_SLAB planes per slab of the 2.5-D kernel for the
@@ -482,8 +539,9 @@ int gm_batch_destroy(gm_batch* b) {
   if (b->xfer) (void)hipStreamSynchronize(b->xfer);
   drop_graph(b);
   free_zombies(b);
+  for (const Block& k : b->spare) drop_block(b, k);
   for (auto& s : b->slots)
-    if (s.used) free_slot(s);
+    if (s.used) drop_block(b, s.block);
   if (b->dboxes) (void)hipFree(b->dboxes);
   if (b->dslots) (void)hipFree(b->dslots);
   if (b->ev_launch) (void)hipEventDestroy(b->ev_launch);
@@ -495,6 +553,7 @@ int gm_batch_destroy(gm_batch* b) {
   if (b->herr) (void)hipHostFree(b->herr);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  gm::xfer_release();
   return GM_OK;
 }
 
@@ -555,18 +614,26 @@ int gm_batch_add(gm_batch* b, const gm_params* p, const double* u, double cfl, d
   const size_t nq = (size_t)p->neq;
   const size_t nu = (size_t)g.ncell * nq * b->esize, n3 = (size_t)g.ncell * 3 * b->esize;
   const size_t nw = (size_t)g.ncell * nq * sizeof(double);
-  struct { void** ptr; size_t n; } al[] = {{&s.U, nu}, {&s.Us, nu}, {&s.W, nw}, {&s.E, n3}};
-  for (auto& a : al) {
-    if (hipMalloc(a.ptr, a.n) != hipSuccess) {
-      (void)hipGetLastError();
-      free_slot(s);
-      return bfail(b, GM_ERR_OOM, "device allocation failed");
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  s.block = take_block(b, (int64_t)(up(nu) + up(nw) + up(nu) + n3));
+  if (!s.block.p) return bfail(b, GM_ERR_OOM, "device allocation failed");
+  // until the box is admitted its block goes back on every way out
+  struct Guard {
+    gm_batch* b;
+    Block* k;
+    ~Guard() {
+      if (k) give_block(b, *k);
     }
-    (void)hipMemsetAsync(*a.ptr, 0, a.n, x);
-  }
+  } guard{b, &s.block};
+  s.U = s.block.p;
+  s.W = s.block.p + up(nu);
+  s.Us = (char*)s.W + up(nw);
+  s.E = (char*)s.Us + up(nu);
+  // no kernel ever reads uninitialised memory: the upload fills U and W
+  BHIP(b, hipMemsetAsync(s.Us, 0, up(nu) + n3, x));
   s.bytes = need;
   // upload: host AoS doubles -> staging (partials block) -> SoA state
-  BHIP(b, hipMemcpyAsync(s.W, u, (size_t)g.ncell * nq * sizeof(double), hipMemcpyHostToDevice, x));
+  BHIP(b, gm::copy_h2d(x, s.W, u, (size_t)g.ncell * nq * sizeof(double)));
   if (b->esize == 8) gm::launch_aos_to_soa(x, g.ncell, (const double*)s.W, (double*)s.U, (int)nq);
   else gm::launch_aos_to_soa(x, g.ncell, (const double*)s.W, (float*)s.U, (int)nq);
   BHIP(b, hipGetLastError());
@@ -588,6 +655,7 @@ int gm_batch_add(gm_batch* b, const gm_params* p, const double* u, double cfl, d
   else gm::launch_cfl_clock(x, box_view<float>(s, slot), &b->dclk[slot].dtmin, b->derr, gm::column_shape(g));
   BHIP(b, hipGetLastError());
   BHIP(b, hipStreamSynchronize(x));
+  guard.k = nullptr;
   s.used = true;
   s.clock = c;
   b->slots[slot] = s;
@@ -612,13 +680,8 @@ int gm_batch_remove(gm_batch* b, int32_t id) {
   BHIP(b, hipStreamSynchronize(b->xfer));
   b->used -= b->slots[id].bytes;
   Slot& sl = b->slots[id];
-  if (b->in_flight) {  // freeing could wait for the launches in flight
-    for (void* q : {sl.U, sl.Us, sl.W, sl.E})
-      if (q) b->zombies.push_back(q);
-    sl = Slot();
-  } else {
-    free_slot(sl);
-  }
+  give_block(b, sl.block);
+  sl = Slot();
   b->tables_dirty = true;
   b->graph_dirty = true;
   return GM_OK;
@@ -709,8 +772,7 @@ int gm_batch_download_u(gm_batch* b, int32_t id, double* u) {
     gm::launch_soa_to_aos(x, g.ncell, (const float*)s.U, (double*)s.W, s.p.neq);
   }
   BHIP(b, hipGetLastError());
-  BHIP(b, hipMemcpyAsync(u, s.W, (size_t)g.ncell * s.p.neq * sizeof(double), hipMemcpyDeviceToHost, x));
-  BHIP(b, hipStreamSynchronize(x));
+  BHIP(b, gm::copy_d2h(x, u, s.W, (size_t)g.ncell * s.p.neq * sizeof(double)));
   return GM_OK;
 }
 

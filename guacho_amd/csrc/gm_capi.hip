@@ -20,6 +20,7 @@
 #include "gm_kernels.hpp"
 #include "guacho_amd.h"
 #include "guacho_amd_user.h"
+#include "gm_xfer.hpp"
 
 namespace {
 
@@ -292,6 +293,7 @@ void release(gm_ctx* c) {
   if (c->hscal) (void)hipHostFree(c->hscal);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
+  gm::xfer_release();
 }
 
 int set_device(gm_ctx* c) { return hip_check(c, hipSetDevice(c->p.device), "hipSetDevice"); }
@@ -710,6 +712,7 @@ int gm_create(const gm_params* params, gm_ctx** out) {
   int rc = validate(params);
   if (rc != GM_OK) return rc;
   gm_ctx* c = new gm_ctx();
+  gm::xfer_retain();  // released with the context
   c->p = *params;
   gm::Geom& g = c->g;
   g.nx = params->nx; g.ny = params->ny; g.nz = params->nz;
@@ -789,7 +792,7 @@ int gm_upload_u(gm_ctx* c, const double* u) {
   c->pc_live = false;  // the host's calcprim of the new state
   const int nq = c->p.neq;
   const size_t n8 = (size_t)c->g.ncell * nq * sizeof(double);
-  GM_HIP(c, hipMemcpyAsync(c->W, u, n8, hipMemcpyHostToDevice, c->stream));
+  GM_HIP(c, gm::copy_h2d(c->stream, c->W, u, n8));
   timed(c, KC_LAYOUT, [&] {
     if (c->esize == 8) gm::launch_aos_to_soa(c->stream, c->g.ncell, (const double*)c->W, (double*)c->U, nq);
     else gm::launch_aos_to_soa(c->stream, c->g.ncell, (const double*)c->W, (float*)c->U, nq);
@@ -822,8 +825,7 @@ int gm_download_u(gm_ctx* c, double* u) {
     else gm::launch_soa_to_aos(c->stream, c->g.ncell, (const float*)c->U, (double*)c->W, nq);
   });
   GM_HIP(c, hipGetLastError());
-  GM_HIP(c, hipMemcpyAsync(u, c->W, (size_t)c->g.ncell * nq * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  GM_HIP(c, hipStreamSynchronize(c->stream));
+  GM_HIP(c, gm::copy_d2h(c->stream, u, c->W, (size_t)c->g.ncell * nq * sizeof(double)));
   return GM_OK;
 }
 
@@ -843,11 +845,8 @@ int gm_download_primit(gm_ctx* c, double* primit, double* temp) {
     else gm::launch_prim_all(c->stream, c->g.ncell, c->ph, (const float*)c->U, (double*)c->W, T, nq, c->g, pc);
   });
   GM_HIP(c, hipGetLastError());
-  GM_HIP(c, hipMemcpyAsync(primit, c->W, (size_t)c->g.ncell * nq * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-  if (temp)
-    GM_HIP(c, hipMemcpyAsync(temp, T, (size_t)c->g.ncell * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  GM_HIP(c, hipStreamSynchronize(c->stream));
+  GM_HIP(c, gm::copy_d2h(c->stream, primit, c->W, (size_t)c->g.ncell * nq * sizeof(double)));
+  if (temp) GM_HIP(c, gm::copy_d2h(c->stream, temp, T, (size_t)c->g.ncell * sizeof(double)));
   return GM_OK;
 }
 
@@ -862,8 +861,7 @@ int gm_download_divb(gm_ctx* c, double* divb) {
   else gm::launch_divb(c->stream, c->g, (const float*)c->U, c->p.dx, c->p.dy, c->p.dz, D);
   GM_HIP(c, hipGetLastError());
   const size_t n = (size_t)c->g.nx * c->g.ny * c->g.nz;
-  GM_HIP(c, hipMemcpyAsync(divb, D, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  GM_HIP(c, hipStreamSynchronize(c->stream));
+  GM_HIP(c, gm::copy_d2h(c->stream, divb, D, n * sizeof(double)));
   return GM_OK;
 }
 

@@ -1,0 +1,22 @@
+// gm_xfer.hpp -- copies between pageable host arrays and device memory.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace gm {
+
+// Keep the staging buffers for as long as some context or batch exists:
+// every context and batch retains once and releases once; the last release
+// frees them.
+void xfer_retain();
+void xfer_release();
+
+// src (pageable host memory) to dst (device memory), ordered on s; src may
+// be changed once the call returns.
+hipError_t copy_h2d(hipStream_t s, void* dst, const void* src, size_t n);
+// src (device memory) to dst (pageable host memory), after the work queued
+// on s; complete when the call returns.
+hipError_t copy_d2h(hipStream_t s, void* dst, const void* src, size_t n);
+
+}  // namespace gm
