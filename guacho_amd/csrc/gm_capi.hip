@@ -126,9 +126,9 @@ namespace {
 // 0: two-kernel) and GUACHO_AMD_SLAB_STAGES ("1", "2", "12": the stages
 // that use the slab kernel) override the choice.
 void stage_policy(int precision, const gm::Geom& g, int kslab[2]) {
-  // slab workgroups resident at once: two per CU in FP64 (256 VGPRs), three
-  // in the mixed form (the FP32 slab kernels hold 154 and 190)
-  const int k = gm::slab_kchunk(g, precision == GM_PRECISION_MIXED ? 768 : 512);
+  // slab workgroups resident at once: two per CU in FP64 (256 VGPRs), four
+  // in the mixed form (128)
+  const int k = gm::slab_kchunk(g, precision == GM_PRECISION_MIXED ? 1024 : 512);
   kslab[0] = g.npas == 0 ? k : 0;
   // a grid whose corrector tiles (32 x 16 x 1) do not reach two per CU runs
   // the corrector as a slab kernel too: one kernel instead of two, and the
@@ -137,7 +137,7 @@ void stage_policy(int precision, const gm::Geom& g, int kslab[2]) {
   // 0.066 against 0.096, 32^3 0.092 against 0.193, 64^3 0.137 against
   // 0.209; 128^3 and up unchanged.
   const long long xy_tiles = (long long)((g.nx + 31) / 32) * ((g.ny + 15) / 16) * g.nz;
-  kslab[1] = (g.npas == 0 && xy_tiles <= 512) ? k : 0;
+  kslab[1] = (g.npas == 0 && (xy_tiles <= 512 || precision == GM_PRECISION_MIXED)) ? k : 0;
   int len = k;
   if (const char* e = std::getenv("GUACHO_AMD_SLAB_KCHUNK")) {
     const long v = std::strtol(e, nullptr, 10);

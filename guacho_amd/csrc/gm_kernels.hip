@@ -16,6 +16,8 @@
 // edge or corner ghost, so a per-axis mapping is exact.
 #include "gm_kernels.hpp"
 
+#include <cmath>
+
 #ifndef GM_KERNELS_PART
 #define GM_KERNELS_PART 0
 #endif
@@ -1023,7 +1025,8 @@ __device__ __forceinline__ void slab_body(const Box<S>& b, unsigned lb, double d
   constexpr int H = L::H, RX = L::RX, PS = L::PS;
   constexpr int NH = FLUXCD ? 5 : 8;
   constexpr bool INC = sizeof(S) == 4;  // mixed: FP32 x/y flux increments
-  static_assert(L::NLOAD <= 2 * SL_THREADS, "two halo loads per thread");
+  constexpr int NHALO = 2 * H * (TYT + TX), HALO0 = SL_THREADS - NHALO;
+  static_assert(HALO0 >= 0, "one halo cell a thread");
   const Geom& g = b.g;
   const int ntx = (g.nx + TX - 1) / TX, nty = (g.ny + TYT - 1) / TYT;
   const unsigned per_plane = (unsigned)(ntx * nty);
@@ -1198,70 +1201,52 @@ __device__ __forceinline__ void slab_body(const Box<S>& b, unsigned lb, double d
     const bool own = c < wx && r < wy;
     const long long col = col_of(tid, own);
     const int at = (r + H) * RX + c + H;  // own cell in the primitive area
-    // the next cell of the window (P(m+ORDER)), the own cell into the
-    // primitive area, the halo (and, in a partial tile, the cells past its
-    // edge) from HBM; ghosts by boundary mapping
+    // the halo (and, in a partial tile, the cells past its edge) and the next
+    // cell of the window (P(m+ORDER)) from HBM, ghosts by boundary mapping.
+    // The halo's 2 H (TYT + TX) cells go to the lanes from HALO0 on, one each:
+    // the x halo of the tile's rows, then the y halo of its columns.  (Found by
+    // walking all cells of tile and halo, the recovery ran in six wavefronts
+    // with a few lanes each instead of two: 256^3 FP64 predictor 1416 us
+    // against 1279, corrector 1995 against 1890; mixed 770 against 683, 1266
+    // against 940.)
+    __builtin_amdgcn_s_setprio(3);
+    S uh[NQ];
+    bool hfx = false, hfy = false;
+    int hx = 0, hy = 0;  // place in the primitive area
+    bool halo = false;
+    {
+      int h = tid - HALO0;
+      if (h >= 0 && h < 2 * H * TYT) {
+        const int s = h / TYT;
+        hx = s < H ? s : wx + s;
+        hy = H + h - s * TYT;
+        halo = hy < H + wy;
+      } else if (h >= 0 && h < NHALO) {
+        h -= 2 * H * TYT;
+        const int s = h / TX;
+        hx = H + h - s * TX;
+        hy = s < H ? s : wy + s;
+        halo = hx < H + wx;
+      }
+      if (halo) {
+        const int si = ghost_src(g, i0 - H + hx, g.nx, g.bc[0], g.bc[1], hfx);
+        const int sj = ghost_src(g, j0 - H + hy, g.ny, g.bc[2], g.bc[3], hfy);
+        const long long hc = cidx(g, si, sj, m);
+#pragma unroll
+        for (int q = 0; q < NQ; q++) uh[q] = Usrc[q * N + hc];
+      }
+    }
     S un[NQ];
     bool unf = false;
     if (own) fetch(col, m + ORDER, un, unf);
+    __builtin_amdgcn_s_setprio(0);
+    // the own cell into the primitive area
     if (own) {
       S pm[NQ];
       wget(tid, m & 1, pm);
 #pragma unroll
       for (int q = 0; q < NQ; q++) lp[q * PS + at] = pm[q];
       if constexpr (ORDER == 1) put_speeds(at, pm, true, true);
-    }
-    __builtin_amdgcn_s_setprio(3);
-    {
-      double u[2][NQ];
-      int dst[2];
-#pragma unroll
-      for (int it = 0; it < 2; it++) {
-        const int idx = tid + it * SL_THREADS;
-        int rx, ry;
-        if (idx < H * TX) {
-          ry = idx / TX;
-          rx = H + idx % TX;
-        } else if (idx < H * TX + TYT * RX) {
-          const int t = idx - H * TX;
-          ry = H + t / RX;
-          rx = t % RX;
-        } else {
-          const int t = idx - H * TX - TYT * RX;
-          ry = H + TYT + t / TX;
-          rx = H + t % TX;
-        }
-        const bool own_pos = rx >= H && rx < H + wx && ry >= H && ry < H + wy;
-        dst[it] = -1;
-        if (idx < L::NLOAD && rx < wx + 2 * H && ry < wy + 2 * H && !own_pos) {
-          dst[it] = ry * RX + rx;
-          load_cons<NQ>(g, Usrc, i0 - H + rx, j0 - H + ry, m, u[it]);
-        }
-      }
-      __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-      for (int it = 0; it < 2; it++) {
-        if (dst[it] < 0) continue;
-        double p[NQ];
-        u2prim<NQ>(b.ph, u[it], p);
-        if (ORDER == 1 && b.pc) {  // Box::pc: interior cells only
-          const int hi = i0 - H + dst[it] % RX, hj = j0 - H + dst[it] / RX;
-          if (hi >= 1 && hi <= g.nx && hj >= 1 && hj <= g.ny) p[4] = b.pc[cidx(g, hi, hj, m)];
-        }
-        S ps[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; q++) {
-          ps[q] = (S)p[q];
-          lp[q * PS + dst[it]] = ps[q];
-        }
-        // a halo cell on one of the tile's rows closes an x face, any other
-        // a y face
-        if constexpr (ORDER == 1) {
-          const int hy = dst[it] / RX;
-          const bool xs = hy >= H && hy < H + wy;
-          put_speeds(dst[it], ps, xs, !xs);
-        }
-      }
     }
     // z face m (above the own cell): P(m) from the window slot, P(m+ORDER)
     // just fetched; the window moves up one cell
@@ -1278,6 +1263,31 @@ __device__ __forceinline__ void slab_body(const Box<S>& b, unsigned lb, double d
       } else {
         z_face(tid, pm, 0, pn, ff);
         wput(tid, (m + 1) & 1, pn);
+      }
+    }
+    if (halo) {
+      double u[NQ], p[NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; q++) u[q] = (double)uh[q];
+      if (hfx) u[1] = -u[1];
+      if (hfy) u[2] = -u[2];
+      u2prim<NQ>(b.ph, u, p);
+      if (ORDER == 1 && b.pc) {  // Box::pc: interior cells only
+        const int hi = i0 - H + hx, hj = j0 - H + hy;
+        if (hi >= 1 && hi <= g.nx && hj >= 1 && hj <= g.ny) p[4] = b.pc[cidx(g, hi, hj, m)];
+      }
+      S ps[NQ];
+      const int hat = hy * RX + hx;
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        ps[q] = (S)p[q];
+        lp[q * PS + hat] = ps[q];
+      }
+      // a halo cell on one of the tile's rows closes an x face, any other
+      // a y face
+      if constexpr (ORDER == 1) {
+        const bool xs = hy >= H && hy < H + wy;
+        put_speeds(hat, ps, xs, !xs);
       }
     }
     __syncthreads();
@@ -2048,12 +2058,14 @@ k_z(Box<S> b, double dt, int kchunk, int* err) {
   z_body<SOLVER, ORDER, FLUXCD, S, NP, W8>(b, gridDim.x - 1 - xcd_logical_block(), dt, kchunk, err);
 }
 
-// the 2.5-D stage kernel: up to 256 VGPRs (two waves per SIMD, two
+// the 2.5-D stage kernel.  FP64: up to 256 VGPRs (two waves per SIMD, two
 // workgroups per CU) for the column window carried across the plane march;
-// the FP64 corrector with passive scalars needs more LDS than two
-// workgroups per CU leave, so it runs at one (the compiler says so)
+// the corrector with passive scalars needs more LDS than two workgroups per
+// CU leave, so it runs at one (the compiler says so).  Mixed: 128 VGPRs, four
+// workgroups per CU (256^3: predictor 683 us at three, 605 at four; corrector
+// 940 and 854, with a 12-byte spill a lane).
 template <int SOLVER, int ORDER, int FLUXCD, typename S, int NP>
-__global__ void __launch_bounds__(SL_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(SL_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(S) == 4 && NP == 0 ? 4 : 2)))
 k_slab(Box<S> b, double dt, int kchunk, int* err) {
   __shared__ S lds[SlabLds<ORDER, 8 + NP, S>::SIZE];
   slab_body<SOLVER, ORDER, FLUXCD, S, NP>(b, xcd_logical_block(), dt, kchunk, err, lds);
@@ -2129,7 +2141,7 @@ kb_xy(const Box<S>* __restrict__ boxes, const unsigned* __restrict__ prefix, int
 // (the FP64 corrector with passive scalars runs at one workgroup per CU,
 // as k_slab does)
 template <int SOLVER, int ORDER, int FLUXCD, typename S, int NP>
-__global__ void __launch_bounds__(SL_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(SL_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(S) == 4 && NP == 0 ? 4 : 2)))
 kb_slab(const Box<S>* __restrict__ boxes, const unsigned* __restrict__ prefix, int nbox,
         const BoxClock* __restrict__ clk, int kchunk, int* err) {
   __shared__ S lds[SlabLds<ORDER, 8 + NP, S>::SIZE];
@@ -2446,33 +2458,27 @@ unsigned slab_tiles(const Geom& g, int kchunk) {
   return ceil_div(g.nx, TX) * ceil_div(g.ny, TYS) * ceil_div(g.nz, kchunk);
 }
 
-// z-planes per slab.  About 2048 workgroups (eight per CU, so the launch's
-// tail is short): at 256^3 that is 32 planes per slab, and 8 to 64 run
-// within 1%; at 96^3 to 192^3, 2 to 13 planes, within 2% of the best length
-// swept.  A grid of no more than two rounds of resident workgroups at one
-// plane per slab (`resident`: the slab workgroups the GPU holds at once,
-// two per CU in FP64, three in the mixed form) does not keep the GPU busy
-// for long, and there the length k minimises
-//   ceil(workgroups(k) / resident) * (k + 1),
-// the rounds of resident workgroups times a workgroup's march (k planes
-// plus about one plane of window warm-up): one round of one- or two-plane
-// marches rather than a second, nearly empty, round.  Per step against the
-// former choice (at least 8 planes per slab): 128x128x4 0.077 ms against
-// 0.108, 1024x4x4 0.066 against 0.096, 32^3 0.092 against 0.193, 64^3
-// 0.137 against 0.209.
+// z-planes per slab, k.  `resident`: the slab workgroups the GPU holds at
+// once (two per CU in FP64, four in the mixed form), r = workgroups(k) /
+// resident the rounds of them, and a workgroup's march is k planes and about
+// one of window warm-up.  A grid of more than two rounds at one plane per
+// slab takes the k that minimises
+//   (ceil(r) + r) / 2 * (k + 1) + k / 2:
+// the marches, half of a nearly empty last round, half a march of tail.  At
+// 256^3 every k from 8 to 32 is within 2% (16 chosen); at 200^3 FP64 it takes
+// 10, 726 us a predictor, where 2048 workgroups (17) took 769 and 25 765.
+// A smaller grid does not keep the GPU busy for long; there k minimises
+// ceil(r) * (k + 1): one round of one- or two-plane marches rather than a
+// second, nearly empty, round (128x128x4 0.077 ms a step against 0.108 at
+// eight planes and more, 64^3 0.137 against 0.209).
 int slab_kchunk(const Geom& g, int resident) {
   const long long per_plane = (long long)ceil_div(g.nx, TX) * ceil_div(g.ny, TYS);
-  if (per_plane * g.nz > 2LL * resident) {
-    long long nslab = (2048 + per_plane - 1) / per_plane;
-    if (nslab > g.nz) nslab = g.nz;
-    if (nslab < 1) nslab = 1;
-    return (int)((g.nz + nslab - 1) / nslab);
-  }
+  const bool large = per_plane * g.nz > 2LL * resident;
   int best = 1;
-  long long best_cost = -1;
-  for (int k = 1; k <= g.nz; k++) {
-    const long long wg = per_plane * ((g.nz + k - 1) / k);
-    const long long cost = ((wg + resident - 1) / resident) * (k + 1);
+  double best_cost = -1.0;
+  for (int k = 1; k <= g.nz && k <= 64; k++) {
+    const double r = (double)(per_plane * ((g.nz + k - 1) / k)) / resident;
+    const double cost = large ? 0.5 * (std::ceil(r) + r) * (k + 1) + 0.5 * k : std::ceil(r) * (k + 1);
     if (best_cost < 0 || cost < best_cost) {
       best_cost = cost;
       best = k;
