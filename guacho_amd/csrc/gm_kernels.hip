@@ -2039,10 +2039,14 @@ __device__ __forceinline__ void cfl_body(const Box<S>& b, unsigned lb, int kchun
 // ---------------------------------------------------------------------------
 // __global__ wrappers: one box ...
 // ---------------------------------------------------------------------------
-// NP passive scalars: their larger LDS tile leaves one workgroup per CU, so
-// the register budget is not squeezed for them.
+// Four waves per SIMD (two workgroups of 8 waves a CU) where the LDS tile
+// allows two workgroups: with one FP64 passive scalar (81,792 bytes) that
+// costs 11 spilled registers a lane and the 120^3 corrector still takes 170 us
+// against 195 at one workgroup.  Two FP64 scalars leave one workgroup per CU,
+// so their register budget is not squeezed.
+constexpr int xy_waves(int np, int esize) { return np == 2 && esize == 8 ? 2 : 4; }
 template <int SOLVER, int ORDER, int FLUXCD, typename S, int NP>
-__global__ void __launch_bounds__(XY_THREADS) __attribute__((amdgpu_waves_per_eu(NP == 0 ? 4 : 2)))
+__global__ void __launch_bounds__(XY_THREADS) __attribute__((amdgpu_waves_per_eu(xy_waves(NP, (int)sizeof(S)))))
 k_xy(Box<S> b, double dt, int* err) {
   __shared__ S lds[XYLds<ORDER, 8 + NP>::SIZE];
   xy_body<SOLVER, ORDER, FLUXCD, S, NP>(b, xcd_logical_block(), dt, err, lds);
@@ -2127,7 +2131,7 @@ __device__ __forceinline__ double stage_dt(const BoxClock* __restrict__ clk, int
 
 // batched kernels: NP passive scalars per box (one count per batch)
 template <int SOLVER, int ORDER, int FLUXCD, typename S, int NP>
-__global__ void __launch_bounds__(XY_THREADS) __attribute__((amdgpu_waves_per_eu(NP == 0 ? 4 : 2)))
+__global__ void __launch_bounds__(XY_THREADS) __attribute__((amdgpu_waves_per_eu(xy_waves(NP, (int)sizeof(S)))))
 kb_xy(const Box<S>* __restrict__ boxes, const unsigned* __restrict__ prefix, int nbox,
       const BoxClock* __restrict__ clk, int* err) {
   __shared__ S lds[XYLds<ORDER, 8 + NP>::SIZE];
