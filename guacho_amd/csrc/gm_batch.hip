@@ -446,15 +446,7 @@ bool valid_id(const gm_batch* b, int32_t id) {
 template <typename S>
 void ghost_fill_t(hipStream_t st, const Slot& s) {
   const gm::Geom g = geom_of(s.p);
-  S* U = (S*)s.U;
-  for (int a = 0; a < 3; a++)
-    if (g.bc[2 * a] == GM_BC_PERIODIC) {
-      gm::launch_ghost(st, g, U, a, 0, GM_BC_PERIODIC, 1);
-      gm::launch_ghost(st, g, U, a, 1, GM_BC_PERIODIC, 1);
-    }
-  for (int kind : {GM_BC_CLOSED, GM_BC_OUTFLOW})
-    for (int f = 0; f < 6; f++)
-      if (g.bc[f] == kind) gm::launch_ghost(st, g, U, f / 2, f % 2, kind, 1);
+  gm::launch_ghost(st, g, (S*)s.U, 1);
 }
 
 }  // namespace

@@ -362,16 +362,8 @@ void user_bc(gm_ctx* c, void* u, int order) {
 // (src/boundaries.f90:245).
 template <typename S>
 void fill_ghost_t(gm_ctx* c, S* U, int layers) {
-  const gm::Geom& g = c->g;
   timed(c, KC_GHOST, [&] {
-    for (int a = 0; a < 3; a++)
-      if (g.bc[2 * a] == GM_BC_PERIODIC) {
-        gm::launch_ghost(c->stream, g, U, a, 0, GM_BC_PERIODIC, layers);
-        gm::launch_ghost(c->stream, g, U, a, 1, GM_BC_PERIODIC, layers);
-      }
-    for (int kind : {GM_BC_CLOSED, GM_BC_OUTFLOW})
-      for (int f = 0; f < 6; f++)
-        if (g.bc[f] == kind) gm::launch_ghost(c->stream, g, U, f / 2, f % 2, kind, layers);
+    gm::launch_ghost(c->stream, c->g, U, layers);
     user_bc(c, U, layers);
   });
 }

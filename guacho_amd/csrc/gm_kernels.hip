@@ -2285,43 +2285,90 @@ __global__ void kb_clock_dt(BoxClock* clk, const int* __restrict__ slots, int nb
 #endif  // GM_PART(1)
 
 // ---------------------------------------------------------------------------
-// ghost fill of one face of the conserved state, serial branches:
+// ghost fill of the conserved state, the serial branches in their order
+// (periodic x, y, z; then closed left..in; then outflow left..in):
 //   layers 1, boundaryI (src/boundaries.f90:44-247): ghost 0 (n+1); periodic
 //     copies over the full transverse range, closed/outflow over 0..n+1;
 //   layers 2, boundaryII (:256-512): ghosts -1, 0 (n+1, n+2) over the full
 //     transverse range; periodic from n-1, n (1, 2), closed/outflow mirrored
 //     (ghost 0 <- cell 1, ghost -1 <- cell 2).
 // Closed walls negate the normal momentum.
+//
+// One launch for all faces: a ghost cell is followed back through the fills
+// from the last, each at most once, to the cell its value starts from.  No
+// fill writes those cells (n >= 2: they are interior, or ghosts that no
+// branch reaches), so the cells of the launch are independent.  It is
+// bound by its launch (9 us with the events around it at 96^3, 8 MB moved); a
+// launch a face took 6 to 12 of 3.0 us each and the gaps between them: a
+// 96^3 conduction step with its two fills took 50 us more, a Brio-Wu run of
+// 50 steps with its one download 4% more.
 // ---------------------------------------------------------------------------
+
+// the fill (axis, side) of `kind` seen backwards: whether it writes cell c
+// (and then c becomes the cell it copies)
+__device__ __forceinline__ bool ghost_back(const Geom& g, int axis, int side, int kind, int layers, int c[3]) {
+  const int n[3] = {g.nx, g.ny, g.nz};
+  const int na = n[axis], lo = (kind == BC_PERIODIC || layers == 2) ? -1 : 0;
+  const int layer = side == 0 ? -c[axis] : c[axis] - na - 1;  // 0: the layer next to the domain
+  if (layer < 0 || layer >= layers) return false;
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+    if (a != axis && (c[a] < lo || c[a] > n[a] + 1 - lo)) return false;
+  if (kind == BC_PERIODIC) c[axis] += side == 0 ? na : -na;
+  else c[axis] = (side == 0 ? 1 : 2 * na + 1) - c[axis];
+  return true;
+}
+
 template <typename S>
-__global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int axis, int side, int kind, int layers) {
-  const int n0 = axis == 0 ? g.ny : g.nx;  // transverse extents (interior)
-  const int n1 = axis == 2 ? g.ny : g.nz;
-  const int na = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
-  const int lo = (kind == BC_PERIODIC || layers == 2) ? -1 : 0;
-  const int e0 = n0 + 2 - 2 * lo, e1 = n1 + 2 - 2 * lo;
-  const long long n = (long long)e0 * e1 * layers;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n;
-       t += (long long)gridDim.x * blockDim.x) {
-    const long long plane = (long long)e0 * e1;
-    const int layer = (int)(t / plane);  // 0: the layer next to the domain
-    const long long r = t - (long long)layer * plane;
-    const int a = (int)(r % e0) + lo;
-    const int b = (int)(r / e0) + lo;
-    const int dst = side == 0 ? -layer : na + 1 + layer;
-    int src;
-    if (kind == BC_PERIODIC) src = side == 0 ? dst + na : dst - na;
-    else src = side == 0 ? 1 - dst : 2 * na + 1 - dst;
-    int di, dj, dk, si, sj, sk;
-    if (axis == 0) { di = dst; si = src; dj = sj = a; dk = sk = b; }
-    else if (axis == 1) { dj = dst; sj = src; di = si = a; dk = sk = b; }
-    else { dk = dst; sk = src; di = si = a; dj = sj = b; }
-    const long long cd = cidx(g, di, dj, dk), cs = cidx(g, si, sj, sk);
-    for (int q = 0; q < 8 + g.npas; q++) {
-      const S v = U[q * g.ncell + cs];
-      U[q * g.ncell + cd] = (kind == BC_CLOSED && q == 1 + axis) ? -v : v;
-    }
+__global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int layers) {
+  // thread to ghost cell: four z planes, then four y rows of the interior
+  // planes, then four x columns of the interior rows
+  long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  const long long nzp = 4LL * g.NX * g.NY, nyp = 4LL * g.NX * g.nz, nxp = 4LL * g.ny * g.nz;
+  if (t >= nzp + nyp + nxp) return;
+  int d[3];
+  auto shell = [](int s, int n) { return s < 2 ? s - 1 : n + s - 1; };  // -1, 0, n+1, n+2
+  if (t < nzp) {
+    d[0] = (int)(t % g.NX) - 1;
+    t /= g.NX;
+    d[1] = (int)(t % g.NY) - 1;
+    d[2] = shell((int)(t / g.NY), g.nz);
+  } else if (t < nzp + nyp) {
+    t -= nzp;
+    d[0] = (int)(t % g.NX) - 1;
+    t /= g.NX;
+    d[1] = shell((int)(t & 3), g.ny);
+    d[2] = (int)(t >> 2) + 1;
+  } else {
+    t -= nzp + nyp;
+    d[0] = shell((int)(t & 3), g.nx);
+    t >>= 2;
+    d[1] = (int)(t % g.ny) + 1;
+    d[2] = (int)(t / g.ny) + 1;
   }
+  int c[3] = {d[0], d[1], d[2]};
+  bool moved = false;
+  int neg = 0;  // bit a: the momentum along a changes sign
+#pragma unroll
+  for (int f = 5; f >= 0; f--)
+    if (g.bc[f] == BC_OUTFLOW) moved |= ghost_back(g, f / 2, f % 2, BC_OUTFLOW, layers, c);
+#pragma unroll
+  for (int f = 5; f >= 0; f--)
+    if (g.bc[f] == BC_CLOSED && ghost_back(g, f / 2, f % 2, BC_CLOSED, layers, c)) {
+      moved = true;
+      neg ^= 1 << (f / 2);
+    }
+#pragma unroll
+  for (int f = 5; f >= 0; f--)
+    if (g.bc[2 * (f / 2)] == BC_PERIODIC) moved |= ghost_back(g, f / 2, f % 2, BC_PERIODIC, layers, c);
+  if (!moved) return;
+  const long long cd = cidx(g, d[0], d[1], d[2]), cs = cidx(g, c[0], c[1], c[2]);
+  S v[10];
+#pragma unroll
+  for (int q = 0; q < 10; q++) v[q] = has_var(q, g.npas) ? U[q * g.ncell + cs] : S(0);
+#pragma unroll
+  for (int q = 0; q < 10; q++)
+    if (has_var(q, g.npas)) U[q * g.ncell + cd] = (q >= 1 && q <= 3 && ((neg >> (q - 1)) & 1)) ? -v[q] : v[q];
 }
 
 // ---------------------------------------------------------------------------
@@ -2688,11 +2735,9 @@ void launch_clock_dt(hipStream_t s, BoxClock* clk, const int* slots, int nbox, i
 #endif  // GM_PART(1)
 
 template <typename S>
-void launch_ghost(hipStream_t s, const Geom& g, S* U, int axis, int side, int kind, int layers) {
-  const int n0 = axis == 0 ? g.ny : g.nx;
-  const int n1 = axis == 2 ? g.ny : g.nz;
-  const long long n = (long long)(n0 + 4) * (n1 + 4) * layers;
-  hipLaunchKernelGGL(k_ghost<S>, dim3(grid_for(n)), dim3(256), 0, s, g, U, axis, side, kind, layers);
+void launch_ghost(hipStream_t s, const Geom& g, S* U, int layers) {
+  const long long n = g.ncell - (long long)g.nx * g.ny * g.nz;
+  hipLaunchKernelGGL(k_ghost<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, U, layers);
 }
 
 template <typename S>
@@ -2738,7 +2783,7 @@ void launch_divb(hipStream_t s, const Geom& g, const S* U, double dx, double dy,
   template void launch_viscous<S>(hipStream_t, const Box<S>&, double);                                            \
   template void launch_tc_dtmin<S>(hipStream_t, const Box<S>&, const Conduction&, const MinOut&);                 \
   template void launch_tc_substep<S>(hipStream_t, const Box<S>&, const Conduction&, double);                      \
-  template void launch_ghost<S>(hipStream_t, const Geom&, S*, int, int, int, int);                               \
+  template void launch_ghost<S>(hipStream_t, const Geom&, S*, int);                                              \
   template void launch_aos_to_soa<S>(hipStream_t, long long, const double*, S*, int);                             \
   template void launch_soa_to_aos<S>(hipStream_t, long long, const S*, double*, int);                             \
   template void launch_prim_all<S>(hipStream_t, long long, const Phys&, const S*, double*, double*, int,         \

@@ -234,10 +234,10 @@ void launch_clock_begin(hipStream_t s, BoxClock* clk, const int* slots, int nbox
 void launch_clock_dt(hipStream_t s, BoxClock* clk, const int* slots, int nbox, int tuning);
 
 // Layout conversion, ghost fill and diagnostics of one box's state.
-// layers 1: one face of boundaryI (src/boundaries.f90:44-247); layers 2:
-// one face of boundaryII (:256-512), two mirrored layers, full transverse range
+// layers 1: boundaryI (src/boundaries.f90:44-247); layers 2: boundaryII
+// (:256-512), two mirrored layers, full transverse range; every face
 template <typename S>
-void launch_ghost(hipStream_t s, const Geom& g, S* U, int axis, int side, int kind, int layers);
+void launch_ghost(hipStream_t s, const Geom& g, S* U, int layers);
 template <typename S>
 void launch_aos_to_soa(hipStream_t s, long long ncell, const double* A, S* D, int nq = 8);
 template <typename S>
