@@ -479,12 +479,13 @@ void conduction_t(gm_ctx* c, const gm::Box<S>& b, double dt) {
     nsteps = 1;
   }
   c->tc_substeps = nsteps;
+  double dts[200];
+  for (int n = 1; n <= nsteps; n++)
+    dts[n - 1] = super ? (((dt_cond * fstep) * tc_substep(n, nsteps, nu)) / tc.psc) / tc.rsc
+                       : ((dt_hydro / (double)nsteps) / tc.psc) / tc.rsc;
   timed(c, KC_CONDUCTION, [&] {
-    for (int n = 1; n <= nsteps; n++) {
-      const double dts = super ? (((dt_cond * fstep) * tc_substep(n, nsteps, nu)) / tc.psc) / tc.rsc
-                               : ((dt_hydro / (double)nsteps) / tc.psc) / tc.rsc;
-      gm::launch_tc_substep(c->stream, b, tc, dts);
-    }
+    gm::launch_tc_substeps(c->stream, b, tc, dts, nsteps);
+    if (c->ubc_fn) gm::launch_tc_outer(c->stream, b);
   });
 }
 

@@ -1701,13 +1701,25 @@ __global__ void __launch_bounds__(256) k_visc_store(Box<S> b) {
 // sub-step kernels.  Temperatures and primitives come from the stored state
 // (ghosts in memory), T = (p / rho) Tempsc as calcprim gives them.
 // Spitzer coefficients Ksp = 6e-7 T^2.5 (:142-149), Ksp_parl = 9.2181e-7
-// T^2.5, Ksp_perp = 0.30089e33 rho / (B^2 sqrt(T)) rho (:157-178); pow and
-// sqrt are the device's.
+// T^2.5, Ksp_perp = 0.30089e33 rho / (B^2 sqrt(T)) rho (:157-178).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double tc_ksp(double t) { return 6.e-7 * pow(t, 2.5); }
-__device__ __forceinline__ double tc_ksp_parl(double t) { return 9.2181e-7 * pow(t, 2.5); }
+// t^2.5 as t^2 sqrt(t), each with its rounding error carried and added back:
+// within 0.501 units in the last place (20 million operands against 64-bit
+// mantissas; 20 FP64 instructions, where pow, itself
+// within one unit, takes some 200 and was two thirds of a face's flux).
+__device__ __forceinline__ double tc_pow25(double t) {
+  const double s = gm_sqrt(t);
+  const double ds = __builtin_fma(-s, s, t) * (0.5 * __builtin_amdgcn_rsq(t));  // sqrt(t) - s
+  const double h = t * t;
+  const double dh = __builtin_fma(t, t, -h);
+  const double p = h * s;
+  const double r = p + (__builtin_fma(h, s, -p) + (dh * s + h * ds));
+  return (p > 0.0 && p < __builtin_inf()) ? r : p;
+}
+__device__ __forceinline__ double tc_ksp(double t) { return 6.e-7 * tc_pow25(t); }
+__device__ __forceinline__ double tc_ksp_parl(double t) { return 9.2181e-7 * tc_pow25(t); }
 __device__ __forceinline__ double tc_ksp_perp(double t, double d, double b2) {
-  return ((0.30089e+33 * d) / (b2 * __builtin_sqrt(t))) * d;
+  return gm_div(0.30089e+33 * d, b2 * gm_sqrt(t)) * d;
 }
 __device__ __forceinline__ double tc_min(double a, double b) { return (a < b) ? a : b; }
 
@@ -1715,21 +1727,27 @@ struct TcCell {
   double rho, p, t, b[3];
 };
 
-template <typename S>
-__device__ __forceinline__ TcCell tc_cell(const Box<S>& b, const Conduction& tc, int i, int j, int k) {
-  const long long c = cidx(b.g, i, j, k), N = b.g.ncell;
-  double u[10], p[10];
-#pragma unroll
-  for (int q = 0; q < 10; q++) u[q] = has_var(q, b.g.npas) ? (double)b.U[q * N + c] : 0.0;
-  const double te = u2prim_t<10>(b.ph, u, p);
+// conserved variables u (8 + npas, zero above) -> TcCell
+__device__ __forceinline__ TcCell tc_prim(const Phys& ph, const Conduction& tc, const double* u) {
+  double p[10];
+  const double te = u2prim_t<10>(ph, u, p);
   TcCell r;
   r.rho = p[0];
   r.p = p[4];
-  r.t = module_temp(b.ph, te, p, tc.tempsc);
+  r.t = module_temp(ph, te, p, tc.tempsc);
   r.b[0] = p[5];
   r.b[1] = p[6];
   r.b[2] = p[7];
   return r;
+}
+
+template <typename S>
+__device__ __forceinline__ TcCell tc_cell(const Box<S>& b, const Conduction& tc, int i, int j, int k) {
+  const long long c = cidx(b.g, i, j, k), N = b.g.ncell;
+  double u[10];
+#pragma unroll
+  for (int q = 0; q < 10; q++) u[q] = has_var(q, b.g.npas) ? (double)b.U[q * N + c] : 0.0;
+  return tc_prim(b.ph, tc, u);
 }
 
 // The workgroup's minimum m (thread 0's) into a MinRed; see there.  Wave 0
@@ -1785,7 +1803,7 @@ __global__ void __launch_bounds__(256) k_tc_dtmin(Box<S> b, Conduction tc, MinOu
     const int i = (int)(t % g.nx) + 1;
     const long long r = t / g.nx;
     const TcCell cl = tc_cell(b, tc, i, (int)(r % g.ny) + 1, (int)(r / g.ny) + 1);
-    v = cl.rho / tc_ksp(cl.t);
+    v = gm_div(cl.rho, tc_ksp(cl.t));
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = tc_min(v, __shfl_xor(v, off, 64));
@@ -1799,104 +1817,233 @@ __global__ void __launch_bounds__(256) k_tc_dtmin(Box<S> b, Conduction tc, MinOu
   }
 }
 
-// heatfluxes (:189-267) / MHD_heatfluxes (:277-487): the three forward faces
-// of every cell (i, j, k) in 0..n, written to W (f, g, h at components 0..2)
-template <typename S>
-__global__ void __launch_bounds__(256) k_tc_flux(Box<S> b, Conduction tc) {
-  const Geom& g = b.g;
-  const int ex = g.nx + 1, ey = g.ny + 1;
-  const long long n = (long long)ex * ey * (g.nz + 1);
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int i = (int)(t % ex);
-  const long long r = t / ex;
-  const int j = (int)(r % ey), k = (int)(r / ey);
-  const double hh[3] = {b.dx, b.dy, b.dz};
-  const TcCell c0 = tc_cell(b, tc, i, j, k);
-  TcCell nb[3];
-  nb[0] = tc_cell(b, tc, i + 1, j, k);
-  nb[1] = tc_cell(b, tc, i, j + 1, k);
-  nb[2] = tc_cell(b, tc, i, j, k + 1);
-  double out[3];
-  if (tc.kind == 1) {
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const TcCell& c1 = nb[a];
-      if (c0.t == c1.t) {
-        out[a] = 0.;
-        continue;
-      }
-      const double meanp = 0.5 * (c0.p + c1.p);
-      const double meand = 0.5 * (c0.rho + c1.rho);
-      const double meant = 0.5 * (c0.t + c1.t);
-      const double dtg = (c1.t - c0.t) / (hh[a] * tc.rsc);
-      double coef;
-      if (tc.sat) {
-        double cs = __builtin_sqrt((b.ph.gamma * meanp) / meand);
-        cs = tc_min(cs * __builtin_sqrt(tc.vsc2), 3.e10);
-        coef = tc_min(tc_ksp(meant), ((((5. * 0.4) * cs) * meanp) * tc.psc) / __builtin_fabs(dtg));
-      } else {
-        coef = tc_ksp(meant);
-      }
-      out[a] = -((coef * dtg) * 1.);
-    }
+// heatfluxes (:189-267): the flux through the face between c0 and c1, h apart
+__device__ __forceinline__ double tc_face(const Conduction& tc, double gamma, double h, const TcCell& c0,
+                                          const TcCell& c1) {
+  if (c0.t == c1.t) return 0.;
+  const double meanp = 0.5 * (c0.p + c1.p);
+  const double meand = 0.5 * (c0.rho + c1.rho);
+  const double meant = 0.5 * (c0.t + c1.t);
+  const double dtg = gm_div(c1.t - c0.t, h * tc.rsc);
+  double coef;
+  if (tc.sat) {
+    double cs = gm_sqrt(gm_div(gamma * meanp, meand));
+    cs = tc_min(cs * gm_sqrt(tc.vsc2), 3.e10);
+    coef = tc_min(tc_ksp(meant), gm_div((((5. * 0.4) * cs) * meanp) * tc.psc, __builtin_fabs(dtg)));
   } else {
-    const double alpha = 5.0 * 0.3;
-    double bx = c0.b[0], by = c0.b[1], bz = c0.b[2];
-    const double b2 = (bx * bx + by * by) + bz * bz;
-    const double modb = __builtin_sqrt(b2);
-    bx = bx / modb;
-    by = by / modb;
-    bz = bz / modb;
-    const double bsc2 = tc.bsc * tc.bsc;
-    double grad[3], kpar[3], kperp[3], csat[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const TcCell& c1 = nb[a];
-      if (__builtin_fabs(c0.t - c1.t) < 1.0e-14) {
-        grad[a] = 0.0;
-        kpar[a] = 0.0;
-        kperp[a] = 0.0;
-        csat[a] = 0.0;
-        continue;
-      }
-      const double meand = 0.5 * (c0.rho + c1.rho);
-      const double meant = 0.5 * (c0.t + c1.t);
-      if (tc.sat) {
-        const double meanp = 0.5 * (c0.p + c1.p);
-        double cs = __builtin_sqrt((b.ph.gamma * meanp) / meand);
-        cs = tc_min(cs * __builtin_sqrt(tc.vsc2), 3.e10);
-        csat[a] = (alpha * meand) * (cs * (cs * cs));  // cs**3 as the compiler's powi forms it
-      } else {
-        csat[a] = 0.0;
-      }
-      grad[a] = (c1.t - c0.t) / (hh[a] * tc.rsc);
-      kpar[a] = tc_ksp_parl(meant);
-      kperp[a] = tc_ksp_perp(meant, meand * tc.rhosc, b2 * bsc2);
-    }
-    const double bgradt = (bx * grad[0] + by * grad[1]) + bz * grad[2];
-    const double gpar[3] = {bgradt * bx, bgradt * by, bgradt * bz};
-    const double gperp[3] = {grad[0] - gpar[0], grad[1] - gpar[1], grad[2] - gpar[2]};
-    if (!tc.sat) {
-#pragma unroll
-      for (int a = 0; a < 3; a++) out[a] = (-(kpar[a] * gpar[a])) - kperp[a] * gperp[a];
-    } else {
-      const double gperpm = __builtin_sqrt((gperp[0] * gperp[0] + gperp[1] * gperp[1]) + gperp[2] * gperp[2]);
-#pragma unroll
-      for (int a = 0; a < 3; a++)
-        out[a] = (-((1. / (1. / (kpar[a] + 1.e-14) + bgradt / (csat[a] + 1.e-14))) * gpar[a]))
-                 - (1. / (1. / (kperp[a] + 1.e-14) + gperpm / (csat[a] + 1.e-14))) * gperp[a];
-    }
+    coef = tc_ksp(meant);
   }
-  const long long c = cidx(g, i, j, k), N = g.ncell;
-  b.W[c] = out[0];
-  b.W[N + c] = out[1];
-  b.W[2 * N + c] = out[2];
+  return -((coef * dtg) * 1.);
 }
 
-// u(5) = u(5) - dts (df/dx + dg/dy + dh/dz) on the interior (:752-758)
+// MHD_heatfluxes (:277-487): the three forward faces of c0
+__device__ __forceinline__ void tc_faces_mhd(const Conduction& tc, double gamma, const double hh[3], const TcCell& c0,
+                                             const TcCell nb[3], double out[3]) {
+  const double alpha = 5.0 * 0.3;
+  double bx = c0.b[0], by = c0.b[1], bz = c0.b[2];
+  const double b2 = (bx * bx + by * by) + bz * bz;
+  const double modb = gm_sqrt(b2);
+  bx = gm_div(bx, modb);
+  by = gm_div(by, modb);
+  bz = gm_div(bz, modb);
+  const double bsc2 = tc.bsc * tc.bsc;
+  double grad[3], kpar[3], kperp[3], csat[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const TcCell& c1 = nb[a];
+    if (__builtin_fabs(c0.t - c1.t) < 1.0e-14) {
+      grad[a] = 0.0;
+      kpar[a] = 0.0;
+      kperp[a] = 0.0;
+      csat[a] = 0.0;
+      continue;
+    }
+    const double meand = 0.5 * (c0.rho + c1.rho);
+    const double meant = 0.5 * (c0.t + c1.t);
+    if (tc.sat) {
+      const double meanp = 0.5 * (c0.p + c1.p);
+      double cs = gm_sqrt(gm_div(gamma * meanp, meand));
+      cs = tc_min(cs * gm_sqrt(tc.vsc2), 3.e10);
+      csat[a] = (alpha * meand) * (cs * (cs * cs));  // cs**3 as the compiler's powi forms it
+    } else {
+      csat[a] = 0.0;
+    }
+    grad[a] = gm_div(c1.t - c0.t, hh[a] * tc.rsc);
+    kpar[a] = tc_ksp_parl(meant);
+    kperp[a] = tc_ksp_perp(meant, meand * tc.rhosc, b2 * bsc2);
+  }
+  const double bgradt = (bx * grad[0] + by * grad[1]) + bz * grad[2];
+  const double gpar[3] = {bgradt * bx, bgradt * by, bgradt * bz};
+  const double gperp[3] = {grad[0] - gpar[0], grad[1] - gpar[1], grad[2] - gpar[2]};
+  if (!tc.sat) {
+#pragma unroll
+    for (int a = 0; a < 3; a++) out[a] = (-(kpar[a] * gpar[a])) - kperp[a] * gperp[a];
+  } else {
+    const double gperpm = gm_sqrt((gperp[0] * gperp[0] + gperp[1] * gperp[1]) + gperp[2] * gperp[2]);
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+      out[a] = (-(gm_div(1., gm_div(1., kpar[a] + 1.e-14) + gm_div(bgradt, csat[a] + 1.e-14)) * gpar[a]))
+               - gm_div(1., gm_div(1., kperp[a] + 1.e-14) + gm_div(gperpm, csat[a] + 1.e-14)) * gperp[a];
+  }
+}
+
+// An E of the result, on its cell and on the edge copies of it that
+// thermal_bounds (:496-616) leaves in ghosts 0 and n+1 (of all axes; over the
+// periodic copies that it makes first)
 template <typename S>
-__global__ void __launch_bounds__(256) k_tc_update(Box<S> b, double dts) {
+__device__ __forceinline__ void tc_put(const Geom& g, S* __restrict__ E, int i, int j, int k, S e) {
+  const int i0 = i == 1 ? 0 : i, i1 = i == g.nx ? i + 1 : i;
+  const int j0 = j == 1 ? 0 : j, j1 = j == g.ny ? j + 1 : j;
+  const int k0 = k == 1 ? 0 : k, k1 = k == g.nz ? k + 1 : k;
+  for (int kk = k0; kk <= k1; kk++)
+    for (int jj = j0; jj <= j1; jj++)
+      for (int ii = i0; ii <= i1; ii++) E[cidx(g, ii, jj, kk)] = e;
+}
+
+// One sub-step (:735-768): the heat fluxes of E = Ein, u(5) = u(5) - dts
+// (df/dx + dg/dy + dh/dz) into Eout.  A workgroup marches a 32 x 8 tile
+// along z.  Each plane's temperatures, with a ring of one cell around the
+// tile, are recovered once into LDS (two planes of them), one plane ahead of
+// the fluxes, its loads two ahead; every cell's three forward faces are
+// solved once, those of the cells below and left of the tile by the first
+// wavefront, and exchanged through LDS; the lower z face stays in a register.
+// FIRST: Ein is the state's own E, ghosts as stored; otherwise the sub-step
+// before's result, whose ghosts are the edge copies: read as such.  GHOSTS:
+// write the copies too (the last sub-step, into the state).
+// Bound by the arithmetic (at two waves per SIMD: at three the 168 registers
+// spill, no faster) and, on small grids, by the march's latency.  With a launch
+// for the fluxes (four recoveries a cell, through memory), one for the update
+// and 12 for the ghost faces, and pow, a step's conduction took 200 us at
+// 96^3 (three sub-steps and their minimum) and 1.4 ms at 160^3; 101 and 450 now.
+constexpr int TCX = 32, TCY = 8, TCRX = TCX + 2, TCN = TCRX * (TCY + 2);
+template <typename S, bool MHD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_tc_step(Box<S> b, Conduction tc, double dts, const S* __restrict__ Ein,
+                                                 S* __restrict__ Eout, int first, int ghosts, int kchunk) {
+  __shared__ double lt[2][TCN], lr[2][TCN], lp[2][TCN];
+  __shared__ double lf[TCY][TCX + 1], lg[TCY + 1][TCX];
+  const Geom& g = b.g;
+  const int ntx = (g.nx + TCX - 1) / TCX, nty = (g.ny + TCY - 1) / TCY;
+  const int tile = (int)(blockIdx.x % (unsigned)(ntx * nty)), kc = (int)(blockIdx.x / (unsigned)(ntx * nty));
+  const int i0 = (tile % ntx) * TCX + 1, j0 = (tile / ntx) * TCY + 1;
+  const int k0 = kc * kchunk + 1, k1 = min(k0 + kchunk - 1, g.nz);
+  const int tid = (int)threadIdx.x, c = tid & (TCX - 1), r = tid / TCX;
+  const int i = i0 + c, j = j0 + r;
+  const int at = (r + 1) * TCRX + c + 1;
+  const bool in = i <= g.nx + 1 && j <= g.ny + 1;  // a stored cell next to the domain, at most
+  const bool own = i <= g.nx && j <= g.ny;
+  // the ring, 84 cells on the last threads
+  const int h = tid - (256 - 2 * TCRX - 2 * TCY);
+  int hx = 0, hy = 0;
+  if (h >= 0) {
+    if (h < TCRX) hx = h, hy = 0;
+    else if (h < 2 * TCRX) hx = h - TCRX, hy = TCY + 1;
+    else if (h < 2 * TCRX + TCY) hx = 0, hy = h - 2 * TCRX + 1;
+    else hx = TCX + 1, hy = h - 2 * TCRX - TCY + 1;
+  }
+  const int hi = i0 - 1 + hx, hj = j0 - 1 + hy;
+  const bool hin = h >= 0 && hi <= g.nx + 1 && hj <= g.ny + 1;
+  const long long N = g.ncell;
+  auto fetch = [&](int ii, int jj, int kk, double* u) {
+    const long long cc = cidx(g, ii, jj, kk);
+    const long long ce = first ? cc : cidx(g, min(max(ii, 1), g.nx), min(max(jj, 1), g.ny), min(max(kk, 1), g.nz));
+#pragma unroll
+    for (int q = 0; q < 10; q++)
+      u[q] = q == 4 ? (double)Ein[ce] : (has_var(q, g.npas) ? (double)b.U[q * N + cc] : 0.0);
+  };
+  auto put = [&](int kk, int pos, const TcCell& cl) {
+    lt[kk & 1][pos] = cl.t;
+    lr[kk & 1][pos] = cl.rho;
+    lp[kk & 1][pos] = cl.p;
+  };
+  auto get = [&](int kk, int pos) {
+    TcCell cl;
+    cl.t = lt[kk & 1][pos];
+    cl.rho = lr[kk & 1][pos];
+    cl.p = lp[kk & 1][pos];
+    cl.b[0] = cl.b[1] = cl.b[2] = 0.0;
+    return cl;
+  };
+  double ua[10], ub[10];
+#pragma unroll
+  for (int q = 0; q < 10; q++) ua[q] = ub[q] = 0.0;
+  TcCell c0, c1{};
+  double e0, e1 = 0.0, hlow = 0.0;
+  auto stage = [&](int kk) {  // the fetched plane kk into LDS; own cell to c1, e1
+    if (in) {
+      c1 = tc_prim(b.ph, tc, ua);
+      e1 = ua[4];
+      put(kk, at, c1);
+    }
+    if (hin) put(kk, hy * TCRX + hx, tc_prim(b.ph, tc, ub));
+  };
+  auto fetch_plane = [&](int kk) {
+    if (in) fetch(i, j, kk, ua);
+    if (hin) fetch(hi, hj, kk, ub);
+  };
+  fetch_plane(k0 - 1);
+  stage(k0 - 1);
+  fetch_plane(k0);
+  const double hh[3] = {b.dx, b.dy, b.dz}, gamma = b.ph.gamma;
+  for (int k = k0 - 1; k <= k1; k++) {
+    c0 = c1;
+    e0 = e1;
+    stage(k + 1);
+    if (k < k1) fetch_plane(k + 2);
+    __syncthreads();
+    double out[3] = {0.0, 0.0, 0.0};
+    const bool warm = k < k0;  // only the z faces below the first plane
+    if (own) {
+      if constexpr (!MHD) {
+        if (!warm) {
+          out[0] = tc_face(tc, gamma, hh[0], c0, get(k, at + 1));
+          out[1] = tc_face(tc, gamma, hh[1], c0, get(k, at + TCRX));
+        }
+        out[2] = tc_face(tc, gamma, hh[2], c0, c1);
+      } else {
+        const TcCell nb[3] = {get(k, at + 1), get(k, at + TCRX), c1};
+        tc_faces_mhd(tc, gamma, hh, c0, nb, out);
+      }
+    }
+    if (!warm) {
+      lf[r][c + 1] = out[0];
+      lg[r + 1][c] = out[1];
+      // the x faces left of the tile's rows, the y faces below its columns
+      if (tid < TCY + TCX) {
+        const bool isx = tid < TCY;
+        const int li = isx ? i0 - 1 : i0 + tid - TCY, lj = isx ? j0 + tid : j0 - 1;
+        if (li <= g.nx && lj <= g.ny) {
+          const int lat = (lj - j0 + 1) * TCRX + li - i0 + 1;
+          TcCell l0 = get(k, lat);
+          double f;
+          if constexpr (!MHD) {
+            f = tc_face(tc, gamma, isx ? hh[0] : hh[1], l0, get(k, isx ? lat + 1 : lat + TCRX));
+          } else {
+            const long long cl = cidx(g, li, lj, k);
+#pragma unroll
+            for (int a = 0; a < 3; a++) l0.b[a] = (double)b.U[(5 + a) * N + cl];
+            const TcCell nb[3] = {get(k, lat + 1), get(k, lat + TCRX), get(k + 1, lat)};
+            double lo[3];
+            tc_faces_mhd(tc, gamma, hh, l0, nb, lo);
+            f = isx ? lo[0] : lo[1];
+          }
+          if (isx) lf[tid][0] = f;
+          else lg[0][tid - TCY] = f;
+        }
+      }
+    }
+    __syncthreads();
+    if (own && !warm) {
+      const S e = (S)(e0 - dts * ((gm_div(out[0] - lf[r][c], b.dx) + gm_div(out[1] - lg[r][c], b.dy)) + gm_div(out[2] - hlow, b.dz)));
+      if (ghosts) tc_put(g, Eout, i, j, k, e);
+      else Eout[cidx(g, i, j, k)] = e;
+    }
+    hlow = out[2];
+  }
+}
+
+// the E of a single sub-step into the state, with its ghost copies
+template <typename S>
+__global__ void __launch_bounds__(256) k_tc_store(Box<S> b, const S* __restrict__ E) {
   const Geom& g = b.g;
   const long long n = (long long)g.nx * g.ny * g.nz;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1904,35 +2051,7 @@ __global__ void __launch_bounds__(256) k_tc_update(Box<S> b, double dts) {
   const int i = (int)(t % g.nx) + 1;
   const long long r = t / g.nx;
   const int j = (int)(r % g.ny) + 1, k = (int)(r / g.ny) + 1;
-  const long long c = cidx(g, i, j, k), N = g.ncell;
-  const long long sy = g.NX, sz = (long long)g.NX * g.NY;
-  const double* F = b.W;
-  const double* G = b.W + N;
-  const double* H = b.W + 2 * N;
-  const double e = (double)b.U[4 * N + c];
-  b.U[4 * N + c] = (S)(e - dts * (((F[c] - F[c - 1]) / b.dx + (G[c] - G[c - sy]) / b.dy) + (H[c] - H[c - sz]) / b.dz));
-}
-
-// thermal_bounds (:496-616) on E, one face: periodic copies over the full
-// transverse range (periodic != 0), else the edge-cell copy over 0..n+1
-template <typename S>
-__global__ void __launch_bounds__(256) k_tc_bound(Geom g, S* __restrict__ U, int axis, int side, int periodic) {
-  const int n0 = axis == 0 ? g.ny : g.nx;
-  const int n1 = axis == 2 ? g.ny : g.nz;
-  const int na = axis == 0 ? g.nx : axis == 1 ? g.ny : g.nz;
-  const int lo = periodic ? -1 : 0;
-  const int e0 = n0 + 2 - 2 * lo, e1 = n1 + 2 - 2 * lo;
-  const long long n = (long long)e0 * e1;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int a = (int)(t % e0) + lo, bq = (int)(t / e0) + lo;
-  const int dst = side == 0 ? 0 : na + 1;
-  const int src = periodic ? (side == 0 ? na : 1) : (side == 0 ? 1 : na);
-  int di, dj, dk, si, sj, sk;
-  if (axis == 0) { di = dst; si = src; dj = sj = a; dk = sk = bq; }
-  else if (axis == 1) { dj = dst; sj = src; di = si = a; dk = sk = bq; }
-  else { dk = dst; sk = src; di = si = a; dj = sj = bq; }
-  U[4 * g.ncell + cidx(g, di, dj, dk)] = U[4 * g.ncell + cidx(g, si, sj, sk)];
+  tc_put(g, b.U + 4 * g.ncell, i, j, k, E[cidx(g, i, j, k)]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2319,14 +2438,11 @@ __device__ __forceinline__ bool ghost_back(const Geom& g, int axis, int side, in
   return true;
 }
 
-template <typename S>
-__global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int layers) {
-  // thread to ghost cell: four z planes, then four y rows of the interior
-  // planes, then four x columns of the interior rows
-  long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+// ghost cell of linear index t: four z planes, then four y rows of the
+// interior planes, then four x columns of the interior rows; false past the last
+__device__ __forceinline__ bool shell_cell(const Geom& g, long long t, int d[3]) {
   const long long nzp = 4LL * g.NX * g.NY, nyp = 4LL * g.NX * g.nz, nxp = 4LL * g.ny * g.nz;
-  if (t >= nzp + nyp + nxp) return;
-  int d[3];
+  if (t >= nzp + nyp + nxp) return false;
   auto shell = [](int s, int n) { return s < 2 ? s - 1 : n + s - 1; };  // -1, 0, n+1, n+2
   if (t < nzp) {
     d[0] = (int)(t % g.NX) - 1;
@@ -2346,6 +2462,13 @@ __global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int la
     d[1] = (int)(t % g.ny) + 1;
     d[2] = (int)(t / g.ny) + 1;
   }
+  return true;
+}
+
+template <typename S>
+__global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int layers) {
+  int d[3];
+  if (!shell_cell(g, blockIdx.x * (long long)blockDim.x + threadIdx.x, d)) return;
   int c[3] = {d[0], d[1], d[2]};
   bool moved = false;
   int neg = 0;  // bit a: the momentum along a changes sign
@@ -2369,6 +2492,22 @@ __global__ void __launch_bounds__(256) k_ghost(Geom g, S* __restrict__ U, int la
 #pragma unroll
   for (int q = 0; q < 10; q++)
     if (has_var(q, g.npas)) U[q * g.ncell + cd] = (q >= 1 && q <= 3 && ((neg >> (q - 1)) & 1)) ? -v[q] : v[q];
+}
+
+// thermal_bounds' periodic copies of E in ghost cells that its edge copies do
+// not reach (an index in the outer layer); boundaryI leaves them the same, so
+// they are made again only after a boundary hook.
+template <typename S>
+__global__ void __launch_bounds__(256) k_tc_outer(Geom g, S* __restrict__ E) {
+  int d[3];
+  if (!shell_cell(g, blockIdx.x * (long long)blockDim.x + threadIdx.x, d)) return;
+  if (d[0] >= 0 && d[0] <= g.nx + 1 && d[1] >= 0 && d[1] <= g.ny + 1 && d[2] >= 0 && d[2] <= g.nz + 1) return;
+  int c[3] = {d[0], d[1], d[2]};
+  bool moved = false;
+#pragma unroll
+  for (int f = 5; f >= 0; f--)
+    if (g.bc[2 * (f / 2)] == BC_PERIODIC) moved |= ghost_back(g, f / 2, f % 2, BC_PERIODIC, 1, c);
+  if (moved) E[cidx(g, d[0], d[1], d[2])] = E[cidx(g, c[0], c[1], c[2])];
 }
 
 // ---------------------------------------------------------------------------
@@ -2619,28 +2758,50 @@ void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, const
   hipLaunchKernelGGL(k_tc_dtmin<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, tc, out);
 }
 
+// Planes per march of k_tc_step, k: two workgroups a CU at once, r rounds of
+// them, marches of k planes and two of warm-up (the plane below the first and
+// the first's own recovery), half of a nearly empty last round, half a march
+// of tail.  us a step's conduction: 64^3 60 / 67 / 100 at k = 2 / 4 / 8 (2
+// taken), 96^3 124 / 113 / 101 / 131 at 2 / 4 / 8 / 16 (8), 160^3 574 / 498 /
+// 448 / 476 (8), 128^3 anisotropic 511 / 441 / 398 / 377 (8).
 template <typename S>
-void launch_tc_substep(hipStream_t s, const Box<S>& b, const Conduction& tc, double dts) {
-  const Geom& g = b.g;
-  const long long nf = (long long)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
-  hipLaunchKernelGGL(k_tc_flux<S>, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, s, b, tc);
-  const long long ni = (long long)g.nx * g.ny * g.nz;
-  hipLaunchKernelGGL(k_tc_update<S>, dim3((unsigned)((ni + 255) / 256)), dim3(256), 0, s, b, dts);
-  auto bound = [&](int axis, int side, int periodic) {
-    const int n0 = axis == 0 ? g.ny : g.nx;
-    const int n1 = axis == 2 ? g.ny : g.nz;
-    const long long n = (long long)(n0 + 4) * (n1 + 4);
-    hipLaunchKernelGGL(k_tc_bound<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, b.U, axis, side,
-                       periodic);
-  };
-  for (int a = 0; a < 3; a++)
-    if (g.bc[2 * a] == BC_PERIODIC && g.bc[2 * a + 1] == BC_PERIODIC) {
-      bound(a, 0, 1);
-      bound(a, 1, 1);
+int tc_kchunk(const Box<S>& b) {
+  const long long per_plane = (long long)ceil_div(b.g.nx, TCX) * ceil_div(b.g.ny, TCY);
+  int best = 1;
+  double best_cost = -1.0;
+  for (int k = 1; k <= b.g.nz && k <= 32; k++) {
+    const double r = (double)(per_plane * ceil_div(b.g.nz, k)) / 512.0;
+    const double cost = 0.5 * (std::ceil(r) + r) * (k + 2) + 0.5 * k;
+    if (best_cost < 0 || cost < best_cost) {
+      best_cost = cost;
+      best = k;
     }
-  for (int a = 0; a < 3; a++) {
-    bound(a, 0, 0);
-    bound(a, 1, 0);
+  }
+  return best;
+}
+
+template <typename S>
+void launch_tc_substeps(hipStream_t s, const Box<S>& b, const Conduction& tc, const double* dts, int nsteps) {
+  const Geom& g = b.g;
+  // E alternates between the state and two halves of W (free by now); the
+  // last sub-step writes the state, which only the first one reads
+  S* const E = b.U + 4 * g.ncell;
+  S* const buf[2] = {reinterpret_cast<S*>(b.W), reinterpret_cast<S*>(b.W) + g.ncell};
+  const long long per_plane = (long long)ceil_div(g.nx, TCX) * ceil_div(g.ny, TCY);
+  const int kchunk = tc_kchunk(b);
+  const unsigned n = (unsigned)(per_plane * ceil_div(g.nz, kchunk));
+  for (int m = 0; m < nsteps; m++) {
+    const S* in = m == 0 ? E : buf[(m - 1) & 1];
+    const bool last = m > 0 && m == nsteps - 1;
+    S* out = last ? E : buf[m & 1];
+    if (tc.kind == 1)
+      hipLaunchKernelGGL((k_tc_step<S, false>), dim3(n), dim3(256), 0, s, b, tc, dts[m], in, out, m == 0, last, kchunk);
+    else
+      hipLaunchKernelGGL((k_tc_step<S, true>), dim3(n), dim3(256), 0, s, b, tc, dts[m], in, out, m == 0, last, kchunk);
+  }
+  if (nsteps == 1) {
+    const long long ni = (long long)g.nx * g.ny * g.nz;
+    hipLaunchKernelGGL(k_tc_store<S>, dim3((unsigned)((ni + 255) / 256)), dim3(256), 0, s, b, (const S*)buf[0]);
   }
 }
 
@@ -2735,6 +2896,12 @@ void launch_clock_dt(hipStream_t s, BoxClock* clk, const int* slots, int nbox, i
 #endif  // GM_PART(1)
 
 template <typename S>
+void launch_tc_outer(hipStream_t s, const Box<S>& b) {
+  const long long n = b.g.ncell - (long long)b.g.nx * b.g.ny * b.g.nz;
+  hipLaunchKernelGGL(k_tc_outer<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b.g, b.U + 4 * b.g.ncell);
+}
+
+template <typename S>
 void launch_ghost(hipStream_t s, const Geom& g, S* U, int layers) {
   const long long n = g.ncell - (long long)g.nx * g.ny * g.nz;
   hipLaunchKernelGGL(k_ghost<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, U, layers);
@@ -2782,7 +2949,8 @@ void launch_divb(hipStream_t s, const Geom& g, const S* U, double dx, double dy,
   template void launch_cooling<S>(hipStream_t, const Box<S>&, const Cooling&, double);                            \
   template void launch_viscous<S>(hipStream_t, const Box<S>&, double);                                            \
   template void launch_tc_dtmin<S>(hipStream_t, const Box<S>&, const Conduction&, const MinOut&);                 \
-  template void launch_tc_substep<S>(hipStream_t, const Box<S>&, const Conduction&, double);                      \
+  template void launch_tc_outer<S>(hipStream_t, const Box<S>&);                                                   \
+  template void launch_tc_substeps<S>(hipStream_t, const Box<S>&, const Conduction&, const double*, int);          \
   template void launch_ghost<S>(hipStream_t, const Geom&, S*, int);                                              \
   template void launch_aos_to_soa<S>(hipStream_t, long long, const double*, S*, int);                             \
   template void launch_soa_to_aos<S>(hipStream_t, long long, const S*, double*, int);                             \

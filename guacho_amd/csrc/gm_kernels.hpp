@@ -186,10 +186,14 @@ struct Conduction {
 // published through `out`
 template <typename S>
 void launch_tc_dtmin(hipStream_t s, const Box<S>& b, const Conduction& tc, const MinOut& out);
-// one sub-step: heat fluxes of cells 0..n (into W), the E update of the
-// interior with dts, thermal_bounds on E
+// the sub-steps dts[0..nsteps): heat fluxes, the E update of the interior,
+// thermal_bounds on E (W is working space)
 template <typename S>
-void launch_tc_substep(hipStream_t s, const Box<S>& b, const Conduction& tc, double dts);
+void launch_tc_substeps(hipStream_t s, const Box<S>& b, const Conduction& tc, const double* dts, int nsteps);
+// thermal_bounds' part that boundaryI has already made unless a boundary
+// hook ran after it
+template <typename S>
+void launch_tc_outer(hipStream_t s, const Box<S>& b);
 // source terms of step() (src/hydro_solver.f90:115-121): up += dt * s after
 // the stage's update, s from the stage's input state
 template <typename S>
