@@ -94,6 +94,7 @@ struct gm_batch {
   bool graph_dirty = true;
   gm::Shape shape = {256, 16, 16, 0, 0};
   bool tuned = false;
+  bool shape_set = false;  // by GUACHO_AMD_BATCH_SLAB
   double tuned_ms = 0.0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -267,6 +268,24 @@ int rebuild_tables_t(gm_batch* b, const gm::Shape& sh) {
 
 int rebuild_tables(gm_batch* b, const gm::Shape& sh) {
   return b->esize == 8 ? rebuild_tables_t<double>(b, sh) : rebuild_tables_t<float>(b, sh);
+}
+
+// The launch shape of the boxes that the next launch steps, as single boxes
+// of their total work choose theirs.  us a step against two-kernel stages with
+// pencils of 16 everywhere: 10 uneven blasts of up to 96^3 444 against 503
+// mixed (969 against 999 FP64), 24 of up to 64^3 356 against 381 (731 against
+// 759), 6 of up to 48^3 78 against 146 (135 against 193).
+gm::Shape default_shape(const gm_batch* b) {
+  std::vector<gm::Geom> g;
+  for (const Slot& s : b->slots)
+    if (s.used && !s.clock.done) g.push_back(geom_of(s.p));
+  if (g.empty()) return b->shape;
+  gm::Shape sh = gm::column_shape(g.data(), (int)g.size());
+  int kslab[2];
+  gm::stage_slabs(g.data(), (int)g.size(), b->bp.precision == GM_PRECISION_MIXED, kslab);
+  sh.slab = kslab[0];
+  sh.slab_both = kslab[1] ? 1 : 0;
+  return sh;
 }
 
 // Queue `nsteps` batched steps (tuning: dt = 0, clocks untouched).
@@ -469,12 +488,14 @@ int gm_batch_create(const gm_batch_params* bp, gm_batch** out) {
   gm_batch* b = new gm_batch();
   gm::xfer_retain();  // released with the batch
   b->bp = *bp;
-  // stage kernels before (or without) autotuning: the two-kernel stage, or
-  // GUACHO_AMD_BATCH_SLAB planes per slab of the 2.5-D kernel for the
-  // predictor (negative: for both stages)
+  // without autotuning each launch's boxes choose their shape
+  // (default_shape), unless GUACHO_AMD_BATCH_SLAB sets it: planes per slab of
+  // the 2.5-D kernel for the predictor (negative: for both stages; 0: the
+  // two-kernel stage)
   if (const char* e = std::getenv("GUACHO_AMD_BATCH_SLAB")) {
     const long v = std::strtol(e, nullptr, 10);
     if (v >= -(1 << 20) && v <= (1 << 20)) {
+      b->shape_set = true;
       b->shape.slab = (int)(v < 0 ? -v : v);
       b->shape.slab_both = v < 0 ? 1 : 0;
     }
@@ -695,6 +716,7 @@ int gm_batch_advance(gm_batch* b, int32_t nlaunch) {
     if ((rc = autotune(b)) != GM_OK) return rc;
   }
   if (b->tables_dirty) {
+    if (!b->tuned && !b->shape_set) b->shape = default_shape(b);
     if ((rc = rebuild_tables(b, b->shape)) != GM_OK) return rc;
     b->graph_dirty = !graph_matches(b);
   }

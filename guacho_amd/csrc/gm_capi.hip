@@ -110,45 +110,12 @@ struct gm_ctx {
 
 namespace {
 
-// The stage kernels of a step, per stage: planes per slab of the 2.5-D
-// kernel, or 0 for the two-kernel stage (xy plane tiles, then z pencils
-// through W).
-//
-// The first-order predictor is a slab kernel on every grid: FP64 256^3 1.28
-// ms against 1.55 for its two kernels; with passive scalars too (us per
-// step, one scalar: FP64 24^3 65 against 78, 60^3 130 against 139, 120^3 638
-// against 704, 192^3 2377 against 2642; mixed 56 against 66, 102 against
-// 108, 367 against 375, 1322 against 1398; two scalars alike).
-//
-// The limited corrector's slab holds a window of planes in LDS and up to 256
-// registers.  FP64 runs it where the corrector's tiles (32 x 16 x 1) do not
-// reach two a CU - one kernel instead of two, and the two-kernel form's four
-// waves per SIMD need a full GPU (per step 128x128x4 0.077 ms against 0.108,
-// 1024x4x4 0.066 against 0.096, 64^3 0.137 against 0.209) - and where
-// the state is a gigabyte and more, whose extra pass through W the memory
-// feels (step 256^3 3.89 ms against 3.93, 320^3 7.61 against 7.73, 384^3 12.7
-// against 13.1); between these lines the two kernels (192^3 1.82 ms against
-// 1.87, 256x256x128 2.12 against 2.14, 80^3 0.178 against 0.185).  The mixed form fits its window
-// and four waves and runs it on every grid (256^3 0.85 ms against 1.05).
-// With passive scalars the LDS window leaves fewer workgroups a CU (one in
-// FP64): the line is one tile a CU in FP64 (one scalar, us per step: 24^3 55
-// against 65, 40^3 at 240 tiles 78 against 79, 48^3 at 288 113 against 101)
-// and one and a half in the mixed form (48^3 67 against 71, 60^3 at 480 105
-// against 102).
-//
-// GUACHO_AMD_SLAB_KCHUNK (planes per slab; 0: two-kernel) and
+// The stage kernels of a step (gm::stage_slabs).  GUACHO_AMD_SLAB_KCHUNK (planes per slab; 0: two-kernel) and
 // GUACHO_AMD_SLAB_STAGES ("1", "2", "12": the stages that use the slab
 // kernel) override the choice.
 void stage_policy(int precision, const gm::Geom& g, int kslab[2]) {
-  const bool mixed = precision == GM_PRECISION_MIXED;
-  // slab workgroups resident at once: two per CU in FP64 (256 VGPRs), four
-  // in the mixed form (128)
-  const int k = gm::slab_kchunk(g, mixed ? 1024 : 512);
-  kslab[0] = k;
-  const long long xy_tiles = (long long)((g.nx + 31) / 32) * ((g.ny + 15) / 16) * g.nz;
-  const bool both = g.npas == 0 ? mixed || xy_tiles <= 512 || xy_tiles >= 32768 : xy_tiles <= (mixed ? 384 : 256);
-  kslab[1] = both ? k : 0;
-  int len = k;
+  gm::stage_slabs(&g, 1, precision == GM_PRECISION_MIXED, kslab);
+  int len = kslab[0];
   if (const char* e = std::getenv("GUACHO_AMD_SLAB_KCHUNK")) {
     const long v = std::strtol(e, nullptr, 10);
     if (v >= 0 && v <= (1 << 20)) {

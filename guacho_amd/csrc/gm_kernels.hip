@@ -2661,13 +2661,20 @@ unsigned slab_tiles(const Geom& g, int kchunk) {
 // ceil(r) * (k + 1): one round of one- or two-plane marches rather than a
 // second, nearly empty, round (128x128x4 0.077 ms a step against 0.108 at
 // eight planes and more, 64^3 0.137 against 0.209).
-int slab_kchunk(const Geom& g, int resident) {
-  const long long per_plane = (long long)ceil_div(g.nx, TX) * ceil_div(g.ny, TYS);
-  const bool large = per_plane * g.nz > 2LL * resident;
+static int slab_kchunk(const Geom* g, int n, int resident) {
+  long long planes = 0;
+  int nz = 1;
+  for (int i = 0; i < n; i++) {
+    planes += slab_tiles(g[i], 1);
+    nz = std::max(nz, g[i].nz);
+  }
+  const bool large = planes > 2LL * resident;
   int best = 1;
   double best_cost = -1.0;
-  for (int k = 1; k <= g.nz && k <= 64; k++) {
-    const double r = (double)(per_plane * ((g.nz + k - 1) / k)) / resident;
+  for (int k = 1; k <= nz && k <= 64; k++) {
+    long long wg = 0;
+    for (int i = 0; i < n; i++) wg += slab_tiles(g[i], k);
+    const double r = (double)wg / resident;
     const double cost = large ? 0.5 * (std::ceil(r) + r) * (k + 1) + 0.5 * k : std::ceil(r) * (k + 1);
     if (best_cost < 0 || cost < best_cost) {
       best_cost = cost;
@@ -2675,6 +2682,42 @@ int slab_kchunk(const Geom& g, int resident) {
     }
   }
   return best;
+}
+
+// The stage kernels of a step of n boxes, per stage: planes per slab of the 2.5-D
+// kernel, or 0 for the two-kernel stage (xy plane tiles, then z pencils
+// through W).
+//
+// The first-order predictor is a slab kernel on every grid: FP64 256^3 1.28
+// ms against 1.55 for its two kernels; with passive scalars too (us per
+// step, one scalar: FP64 24^3 65 against 78, 60^3 130 against 139, 120^3 638
+// against 704, 192^3 2377 against 2642; mixed 56 against 66, 102 against
+// 108, 367 against 375, 1322 against 1398; two scalars alike).
+//
+// The limited corrector's slab holds a window of planes in LDS and up to 256
+// registers.  FP64 runs it where the corrector's tiles (32 x 16 x 1) do not
+// reach two a CU - one kernel instead of two, and the two-kernel form's four
+// waves per SIMD need a full GPU (per step 128x128x4 0.077 ms against 0.108,
+// 1024x4x4 0.066 against 0.096, 64^3 0.137 against 0.209) - and where
+// the state is a gigabyte and more, whose extra pass through W the memory
+// feels (step 256^3 3.89 ms against 3.93, 320^3 7.61 against 7.73, 384^3 12.7
+// against 13.1); between these lines the two kernels (192^3 1.82 ms against
+// 1.87, 256x256x128 2.12 against 2.14, 80^3 0.178 against 0.185).  The mixed form fits its window
+// and four waves and runs it on every grid (256^3 0.85 ms against 1.05).
+// With passive scalars the LDS window leaves fewer workgroups a CU (one in
+// FP64): the line is one tile a CU in FP64 (one scalar, us per step: 24^3 55
+// against 65, 40^3 at 240 tiles 78 against 79, 48^3 at 288 113 against 101)
+// and one and a half in the mixed form (48^3 67 against 71, 60^3 at 480 105
+// against 102).
+void stage_slabs(const Geom* g, int n, bool mixed, int kslab[2]) {
+  // slab workgroups resident at once: two per CU in FP64 (256 VGPRs), four
+  // in the mixed form (128)
+  const int k = slab_kchunk(g, n, mixed ? 1024 : 512);
+  long long xy_tiles = 0;
+  for (int i = 0; i < n; i++) xy_tiles += (long long)ceil_div(g[i].nx, TX) * ceil_div(g[i].ny, TY) * g[i].nz;
+  const bool both = g[0].npas == 0 ? mixed || xy_tiles <= 512 || xy_tiles >= 32768 : xy_tiles <= (mixed ? 384 : 256);
+  kslab[0] = k;
+  kslab[1] = both ? k : 0;
 }
 #endif  // GM_PART(1)
 
@@ -2730,8 +2773,9 @@ void launch_cfl_clock(hipStream_t s, const Box<S>& b, unsigned long long* dtmin,
 // 43.3 (39.8, 27.8), 150x70x45 44.4 against 30.1 (36.9, 19.9); field update
 // with the CFL minimum 64^3 34.6 against 13.8 (35.9, 12.7), 128x128x4 15.2
 // against 10.4, 113^3 51.7 against 41.9; field update 64^3 16.0 against 9.2.
-Shape column_shape(const Geom& g) {
-  const long long work = (long long)ceil_div((long long)g.nx * g.ny, 256) * g.nz;  // tiles x planes
+Shape column_shape(const Geom* g, int n) {
+  long long work = 0;  // tiles x planes
+  for (int i = 0; i < n; i++) work += (long long)ceil_div((long long)g[i].nx * g[i].ny, 256) * g[i].nz;
   auto clamp = [](long long v, int lo, int hi) { return (int)(v < lo ? lo : v > hi ? hi : v); };
   return Shape{256, clamp((work + 511) / 512, 4, 16), clamp((work + 1023) / 1024, 1, 16), 0, 0};
 }

@@ -96,8 +96,9 @@ struct Shape {
   int slab_both;   // batches: 1 when the corrector runs as the slab kernel too
 };
 
-// the column kernels' shape for one grid
-Shape column_shape(const Geom& g);
+// the column kernels' shape for n boxes stepped together
+Shape column_shape(const Geom* g, int n);
+inline Shape column_shape(const Geom& g) { return column_shape(&g, 1); }
 
 // Minimum over all workgroups of a launch, published by the launch itself.
 // Atomics on one address are serial here at 11.5 ns each (4096 workgroups:
@@ -152,8 +153,10 @@ void launch_z(hipStream_t s, const Box<S>& b, double dt, int stage, int solver, 
 template <typename S>
 void launch_slab(hipStream_t s, const Box<S>& b, double dt, int stage, int solver, int flux_cd, int* err,
                  int kchunk);
-// default slab length for a grid, and the workgroups of a slab launch
-int slab_kchunk(const Geom& g, int resident);
+// the stage kernels of n boxes stepped together (of the same variables): per
+// stage the planes per slab, 0 for the two-kernel stage; and the workgroups
+// of a slab launch
+void stage_slabs(const Geom* g, int n, bool mixed, int kslab[2]);
 unsigned slab_tiles(const Geom& g, int kchunk);
 // `idle`: a MinRed to zero on the way (null: none), for a caller that does
 // not know how the last launch over it ended
