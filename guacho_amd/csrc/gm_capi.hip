@@ -507,13 +507,20 @@ void tstep_t(gm_ctx* c, double dt) {
   stage_sources_t(c, b, dt, 2);
   // viscous_copy (src/hydro_solver.f90:188); with eta = 0 the identity on
   // values, so no pass
-  if (p.eta != 0.0) timed(c, KC_VISCOUS, [&] { gm::launch_viscous(s, b, p.eta); });
+  const bool visc = p.eta != 0.0;
+  if (visc) timed(c, KC_VISCOUS, [&] { gm::launch_viscous(s, b, p.eta); });
   // cooling (src/hydro_solver.f90:206-210); table cooling also leaves the
   // interior cells' primit pressure for the next step (Box::pc)
+  // and, unless conduction or a boundary hook still follows, is the last pass
+  // over the interior: it reduces the next get_timestep's minimum too
   if (c->cool.kind) {
     gm::Box<S> bc = b;
     bc.pc = c->cool.kind == GM_COOL_H ? nullptr : c->Pc;
-    timed(c, KC_COOLING, [&] { gm::launch_cooling(s, bc, c->cool, dt); });
+    const gm::MinOut out = cfl_out(c);
+    c->cfl_pending = !c->cond.kind && !c->ubc_fn;
+    timed(c, KC_COOLING, [&] { gm::launch_finish(s, bc, visc, c->cool, dt, c->cfl_pending ? &out : nullptr); });
+  } else if (visc) {
+    timed(c, KC_VISCOUS, [&] { gm::launch_finish(s, b, true, c->cool, dt, nullptr); });
   }
   // boundaryI on U^{n+1} (src/hydro_solver.f90:216) when ghosts live in memory
   if (b.g.gmem) fill_ghost_t<S>(c, b.U, 1);
@@ -667,8 +674,12 @@ void noalloc_tstep_t(hipStream_t s, const gm_params& p, S* u, const ScratchPtrs&
   } else {
     if (fcd) gm::launch_bfield(s, b, dt, 2, sh);
     if (b.src && !b.srcin) gm::launch_sources(s, b, dt, 2, sh);
-    if (p.eta != 0.0) gm::launch_viscous(s, b, p.eta);
-    gm::launch_cfl(s, b, out, sh);
+    if (p.eta != 0.0) {
+      gm::launch_viscous(s, b, p.eta);
+      gm::launch_finish(s, b, true, gm::Cooling{}, dt, &out);
+    } else {
+      gm::launch_cfl(s, b, out, sh);
+    }
   }
 }
 

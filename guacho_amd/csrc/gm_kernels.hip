@@ -1481,31 +1481,20 @@ __device__ __forceinline__ double cool_lambda(const Cooling& cl, double T) {
   return ((c1 - c0) * (T - T0)) / (T1 - T0) + c0;
 }
 
-template <typename S>
-__global__ void __launch_bounds__(256) k_cooling(Box<S> b, Cooling cl, double dt) {
-  const Geom& g = b.g;
-  const long long n = (long long)g.nx * g.ny * g.nz;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int i = (int)(t % g.nx) + 1;
-  const long long r = t / g.nx;
-  const int j = (int)(r % g.ny) + 1, k = (int)(r / g.ny) + 1;
-  const long long c = cidx(g, i, j, k), N = g.ncell;
-  double u[10], p[10];
-#pragma unroll
-  for (int q = 0; q < 10; q++) u[q] = has_var(q, g.npas) ? (double)b.U[q * N + c] : 0.0;
-  const double T = module_temp(b.ph, u2prim_t<10>(b.ph, u, p), p, cl.tempsc);
-  if (!(T > 10000.)) {
-    if (b.pc) b.pc[c] = p[4];  // primit(5) = u2prim's pressure
-    return;
-  }
-  const double eth0 = b.ph.cv * p[4];
+// one cell: the cooled E into u[4] (true) or u left alone (false); pn: the
+// pressure primit(5) is left with
+__device__ __forceinline__ bool cool_table(const Phys& ph, const Cooling& cl, double dt, double* u, double& pn) {
+  double p[10];
+  const double T = module_temp(ph, u2prim_t<10>(ph, u, p), p, cl.tempsc);
+  pn = p[4];  // u2prim's pressure
+  if (!(T > 10000.)) return false;
+  const double eth0 = ph.cv * p[4];
   const double aloss = cool_lambda(cl, T);
   const double dens = p[0];
   const double ce = (aloss * (dens * dens)) / (eth0 * cl.psc);
-  const double pn = p[4] * exp(-(ce * (dt * cl.tsc)));
-  b.U[4 * N + c] = (S)((u[4] - eth0) + b.ph.cv * pn);
-  if (b.pc) b.pc[c] = pn;  // primit(5), cooled
+  pn = p[4] * exp(-(ce * (dt * cl.tsc)));  // cooled
+  u[4] = (u[4] - eth0) + ph.cv * pn;
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1579,20 +1568,10 @@ __device__ double hr_aloss(double x1, double den, double dh0, double te0) {
   return ((ecoll + eion) + line) + equil * fr;
 }
 
-template <typename S>
-__global__ void __launch_bounds__(256) k_cooling_h(Box<S> b, Cooling cl, double dt) {
-  const Geom& g = b.g;
-  const long long n = (long long)g.nx * g.ny * g.nz;
-  const long long tt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tt >= n) return;
-  const int i = (int)(tt % g.nx) + 1;
-  const long long r = tt / g.nx;
-  const int j = (int)(r % g.ny) + 1, k = (int)(r / g.ny) + 1;
-  const long long c = cidx(g, i, j, k), N = g.ncell;
-  double u[10], p[10];
-#pragma unroll
-  for (int q = 0; q < 10; q++) u[q] = has_var(q, g.npas) ? (double)b.U[q * N + c] : 0.0;
-  const double t = module_temp(b.ph, u2prim_t<10>(b.ph, u, p), p, cl.tempsc);
+// one cell: the cooled E and the neutral density into u[4] and u[8]
+__device__ __forceinline__ void cool_h(const Phys& ph, const Cooling& cl, double dt, double* u) {
+  double p[10];
+  const double t = module_temp(ph, u2prim_t<10>(ph, u, p), p, cl.tempsc);
   const double dts = dt * cl.tsc;
   const double xi = 1.e-4, boltzm = 1.3807e-16;
   const double col = (5.83e-11 * gm_sqrt(t)) * exp(-gm_div(157828., t));
@@ -1615,11 +1594,11 @@ __global__ void __launch_bounds__(256) k_cooling_h(Box<S> b, Cooling cl, double 
   t1 = dmax(t1, 0.1 * t);
   t1 = dmin(t1, 10. * t);
   const double u9 = y1 * u[0];
-  double e5 = gm_div((b.ph.cv * ((2. * u[0]) - u9)) * t1, cl.tempsc)
+  double e5 = gm_div((ph.cv * ((2. * u[0]) - u9)) * t1, cl.tempsc)
               + (0.5 * p[0]) * ((p[1] * p[1] + p[2] * p[2]) + p[3] * p[3]);
-  if (b.ph.mhd) e5 = e5 + 0.5 * ((p[5] * p[5] + p[6] * p[6]) + p[7] * p[7]);
-  b.U[8 * N + c] = (S)u9;
-  b.U[4 * N + c] = (S)e5;
+  if (ph.mhd) e5 = e5 + 0.5 * ((p[5] * p[5] + p[6] * p[6]) + p[7] * p[7]);
+  u[8] = u9;
+  u[4] = e5;
 }
 
 // ---------------------------------------------------------------------------
@@ -1698,16 +1677,6 @@ __global__ void __launch_bounds__(256) k_viscous(Box<S> b, double eta) {
   if (t >= n) return;
   const long long r = t / g.nx;
   visc_cell(b, (int)(t % g.nx) + 1, (int)(r % g.ny) + 1, (int)(r / g.ny) + 1, eta);
-}
-
-template <typename S>
-__global__ void __launch_bounds__(256) k_visc_store(Box<S> b) {
-  const Geom& g = b.g;
-  const long long n = (long long)g.nx * g.ny * g.nz;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const long long r = t / g.nx;
-  visc_store_cell(b, (int)(t % g.nx) + 1, (int)(r % g.ny) + 1, (int)(r / g.ny) + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -2146,6 +2115,51 @@ __device__ __forceinline__ void cfl_reduce(double dtp, bool bad, unsigned long l
     const unsigned long long v = (unsigned long long)__double_as_longlong(m);
     if (v < __hip_atomic_load(dtmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(dtmin, v);
   }
+}
+
+// What follows the corrector cell by cell, in one pass: the viscous result
+// out of W (VISC), cooling (COOL: 0 none, 1 table, 2 H-rate) and, where
+// nothing after it touches the interior, get_timestep's minimum of the result
+// (CFL), on the values as stored.  Bound by its traffic, or by cool_h's
+// arithmetic, under which the minimum's reads are hidden.  A pass each, 128^3
+// with viscosity and table cooling took 47 + 32 + 34 us, 120^3 with H-rate
+// cooling 75 + 31; one takes 60 and 96.
+template <typename S, bool VISC, int COOL, bool CFL>
+__global__ void __launch_bounds__(256) k_finish(Box<S> b, Cooling cl, double dt, MinOut out) {
+  const Geom& g = b.g;
+  const long long n = (long long)g.nx * g.ny * g.nz;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  double dtp = 1e30;
+  bool bad = false;
+  if (t < n) {
+    const int i = (int)(t % g.nx) + 1;
+    const long long r = t / g.nx;
+    const int j = (int)(r % g.ny) + 1, k = (int)(r / g.ny) + 1;
+    const long long c = cidx(g, i, j, k), N = g.ncell;
+    double u[10];
+#pragma unroll
+    for (int q = 0; q < 10; q++)
+      u[q] = has_var(q, g.npas) ? (VISC ? (double)(S)b.W[q * N + c] : (double)b.U[q * N + c]) : 0.0;
+    bool e_new = false;
+    double pn = 0.0;
+    if constexpr (COOL == 1) {
+      e_new = cool_table(b.ph, cl, dt, u, pn);
+      b.pc[c] = pn;  // set with table cooling
+    }
+    if constexpr (COOL == 2) {
+      cool_h(b.ph, cl, dt, u);
+      e_new = true;
+    }
+#pragma unroll
+    for (int q = 0; q < 10; q++) {
+      if (!has_var(q, g.npas)) continue;
+      u[q] = (double)(S)u[q];
+      if (VISC || (q == 4 && e_new) || (q == 8 && COOL == 2)) b.U[q * N + c] = (S)u[q];
+      if (CFL) bad |= !__builtin_isfinite(u[q]);
+    }
+    if constexpr (CFL) dtp = cfl_cell<10, S>(b.ph, b.dx, b.dy, b.dz, u, dtp, COOL == 1 ? &pn : nullptr);
+  }
+  if constexpr (CFL) cfl_reduce(dtp, bad, out);
 }
 
 template <typename S, int NQ = 8>
@@ -2798,16 +2812,27 @@ Shape column_shape(const Geom* g, int n) {
 template <typename S>
 void launch_viscous(hipStream_t s, const Box<S>& b, double eta) {
   const long long n = (long long)b.g.nx * b.g.ny * b.g.nz;
-  const dim3 grid((unsigned)((n + 255) / 256));
-  hipLaunchKernelGGL(k_viscous<S>, grid, dim3(256), 0, s, b, eta);
-  hipLaunchKernelGGL(k_visc_store<S>, grid, dim3(256), 0, s, b);
+  hipLaunchKernelGGL(k_viscous<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, eta);
 }
 
 template <typename S>
-void launch_cooling(hipStream_t s, const Box<S>& b, const Cooling& cl, double dt) {
+void launch_finish(hipStream_t s, const Box<S>& b, bool visc, const Cooling& cl, double dt, const MinOut* cfl) {
   const long long n = (long long)b.g.nx * b.g.ny * b.g.nz;
-  if (cl.kind == GM_COOL_H) hipLaunchKernelGGL(k_cooling_h<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, cl, dt);
-  else hipLaunchKernelGGL(k_cooling<S>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, cl, dt);
+  const dim3 grid((unsigned)((n + 255) / 256));
+  const MinOut out = cfl ? *cfl : MinOut{nullptr, nullptr, nullptr, nullptr, 0};
+#define GM_FINISH(V, C)                                                                            \
+  {                                                                                                \
+    if (cfl) hipLaunchKernelGGL((k_finish<S, V, C, true>), grid, dim3(256), 0, s, b, cl, dt, out); \
+    else hipLaunchKernelGGL((k_finish<S, V, C, false>), grid, dim3(256), 0, s, b, cl, dt, out);    \
+  }
+  if (cl.kind == GM_COOL_H) {
+    if (visc) GM_FINISH(true, 2) else GM_FINISH(false, 2)
+  } else if (cl.kind) {
+    if (visc) GM_FINISH(true, 1) else GM_FINISH(false, 1)
+  } else if (visc) {
+    GM_FINISH(true, 0)
+  }
+#undef GM_FINISH
 }
 
 template <typename S>
@@ -3004,7 +3029,7 @@ void launch_divb(hipStream_t s, const Geom& g, const S* U, double dx, double dy,
   template void launch_cfl_clock<S>(hipStream_t, const Box<S>&, unsigned long long*, int*, const Shape&);         \
   template void launch_bfield_cfl<S>(hipStream_t, const Box<S>&, double, const MinOut&, const Shape&);            \
   template void launch_sources<S>(hipStream_t, const Box<S>&, double, int, const Shape&);                         \
-  template void launch_cooling<S>(hipStream_t, const Box<S>&, const Cooling&, double);                            \
+  template void launch_finish<S>(hipStream_t, const Box<S>&, bool, const Cooling&, double, const MinOut*);        \
   template void launch_viscous<S>(hipStream_t, const Box<S>&, double);                                            \
   template void launch_tc_dtmin<S>(hipStream_t, const Box<S>&, const Conduction&, const MinOut&);                 \
   template void launch_tc_outer<S>(hipStream_t, const Box<S>&);                                                   \

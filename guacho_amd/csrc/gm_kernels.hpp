@@ -172,12 +172,14 @@ void launch_cfl_clock(hipStream_t s, const Box<S>& b, unsigned long long* dtmin,
 // reduction over the updated state
 template <typename S>
 void launch_bfield_cfl(hipStream_t s, const Box<S>& b, double dt, const MinOut& out, const Shape& sh);
-// cooling pass on U^{n+1} (src/hydro_solver.f90:206-210) with the step's dt
-// viscous_copy with eta != 0 (W as scratch), after the corrector
+// viscous_copy with eta != 0 after the corrector, its result into W
 template <typename S>
 void launch_viscous(hipStream_t s, const Box<S>& b, double eta);
+// ... which launch_finish stores (visc), with the cooling pass on U^{n+1}
+// (src/hydro_solver.f90:206-210; kind 0: none) and the step's dt, and, with
+// cfl, launch_cfl's reduction of the result
 template <typename S>
-void launch_cooling(hipStream_t s, const Box<S>& b, const Cooling& cl, double dt);
+void launch_finish(hipStream_t s, const Box<S>& b, bool visc, const Cooling& cl, double dt, const MinOut* cfl);
 
 // Thermal conduction (thermal_cond.f90): kind 1 isotropic, 2 anisotropic;
 // the parameters module's scalings.  Ghosts live in memory while it is on.
