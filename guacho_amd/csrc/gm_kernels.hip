@@ -1669,15 +1669,11 @@ __device__ __forceinline__ void visc_store_cell(const Box<S>& b, int i, int j, i
     if (has_var(q, b.g.npas)) b.U[q * N + c] = (S)b.W[q * N + c];
 }
 
-// Consecutive workgroups on one XCD in the mixed form, whose three planes of
-// neighbours fit its L2 (128^3 53 -> 45 us); in FP64 they do not (109 -> 113),
-// and the XCDs share the planes in flight through the memory-side cache.
 template <typename S>
 __global__ void __launch_bounds__(256) k_viscous(Box<S> b, double eta) {
   const Geom& g = b.g;
   const long long n = (long long)g.nx * g.ny * g.nz;
-  const unsigned lb = sizeof(S) == 4 ? xcd_logical_block() : blockIdx.x;
-  const long long t = (long long)lb * blockDim.x + threadIdx.x;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const long long r = t / g.nx;
   visc_cell(b, (int)(t % g.nx) + 1, (int)(r % g.ny) + 1, (int)(r / g.ny) + 1, eta);
@@ -1901,7 +1897,8 @@ __device__ __forceinline__ void tc_put(const Geom& g, S* __restrict__ E, int i, 
 // spill, no faster) and, on small grids, by the march's latency.  With a launch
 // for the fluxes (four recoveries a cell, through memory), one for the update
 // and 12 for the ghost faces, and pow, a step's conduction took 200 us at
-// 96^3 (three sub-steps and their minimum) and 1.4 ms at 160^3; 101 and 450 now.
+// 96^3 (three sub-steps and their minimum) and 1.4 ms at 160^3; 92 and 425 now
+// (98 and 446 with neighbouring tiles on different XCDs).
 constexpr int TCX = 32, TCY = 8, TCRX = TCX + 2, TCN = TCRX * (TCY + 2);
 template <typename S, bool MHD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_tc_step(Box<S> b, Conduction tc, double dts, const S* __restrict__ Ein,
