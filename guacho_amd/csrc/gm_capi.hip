@@ -110,9 +110,9 @@ struct gm_ctx {
 
 namespace {
 
-// The stage kernels of a step (gm::stage_slabs).  GUACHO_AMD_SLAB_KCHUNK (planes per slab; 0: two-kernel) and
-// GUACHO_AMD_SLAB_STAGES ("1", "2", "12": the stages that use the slab
-// kernel) override the choice.
+// The stage kernels of a step (gm::stage_slabs).  GUACHO_AMD_SLAB_KCHUNK
+// (planes per slab; 0: two-kernel) and GUACHO_AMD_SLAB_STAGES ("1", "2",
+// "12": the stages that use the slab kernel) override the choice.
 void stage_policy(int precision, const gm::Geom& g, int kslab[2]) {
   gm::stage_slabs(&g, 1, precision == GM_PRECISION_MIXED, kslab);
   int len = kslab[0];

@@ -2714,8 +2714,8 @@ static int slab_kchunk(const Geom* g, int n, int resident) {
   return best;
 }
 
-// The stage kernels of a step of n boxes, per stage: planes per slab of the 2.5-D
-// kernel, or 0 for the two-kernel stage (xy plane tiles, then z pencils
+// The stage kernels of a step of n boxes, per stage: planes per slab of the
+// 2.5-D kernel, or 0 for the two-kernel stage (xy plane tiles, then z pencils
 // through W).
 //
 // The first-order predictor is a slab kernel on every grid: FP64 256^3 1.28
@@ -2732,8 +2732,9 @@ static int slab_kchunk(const Geom* g, int n, int resident) {
 // the state is a gigabyte and more, whose extra pass through W the memory
 // feels (step 256^3 3.89 ms against 3.93, 320^3 7.61 against 7.73, 384^3 12.7
 // against 13.1); between these lines the two kernels (192^3 1.82 ms against
-// 1.87, 256x256x128 2.12 against 2.14, 80^3 0.178 against 0.185).  The mixed form fits its window
-// and four waves and runs it on every grid (256^3 0.85 ms against 1.05).
+// 1.87, 256x256x128 2.12 against 2.14, 80^3 0.178 against 0.185).  The mixed
+// form fits its window and four waves and runs it on every grid (256^3 0.85 ms
+// against 1.05).
 // With passive scalars the LDS window leaves fewer workgroups a CU (one in
 // FP64): the line is one tile a CU in FP64 (one scalar, us per step: 24^3 55
 // against 65, 40^3 at 240 tiles 78 against 79, 48^3 at 288 113 against 101)
